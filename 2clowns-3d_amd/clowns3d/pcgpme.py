@@ -142,7 +142,7 @@ class Solver:
 
     def index_bits(self):
         """8 or 16 if the resident operator's kernels read 8- or 16-bit coded
-        neighbour indices, else 32."""
+        neighbour indices, else 32; 0 where they run by row runs."""
         return L.lib().clowns_solver_index_bits(self._h)
 
     def set_block_order(self, order=None):
@@ -161,10 +161,10 @@ class Solver:
         """Kernel forms chosen for the resident operator (clowns_solver_tuning):
         dict fuse64, fuse32 (1 fused PM pairs), stream64, stream32 (bit 0
         streamed PM stages, bit 1 streamed SpMV), index64, index32 (bits of
-        the neighbour-index codes: 8, 16 or 32), pmpat64 (1: FP64 PM stages
+        the neighbour-index codes: 8, 16 or 32; 0: row runs), pmpat64 (1: FP64 PM stages
         with the row-pattern table), spmv32 (FP32 SpMV: 0 column-major, 1
         row-major copies, 2 row-major in two chunks a wavefront, plus 4 with
-        the row-pattern table); -1 where undecided."""
+        the row-pattern table; 8 row runs); -1 where undecided."""
         out = np.zeros(8, np.int32)
         L.check(L.lib().clowns_solver_tuning(self._h, ctypes.c_void_p(out.ctypes.data)), "clowns_solver_tuning")
         return dict(zip(("fuse64", "fuse32", "stream64", "stream32", "index64", "index32", "pmpat64", "spmv32"),

@@ -771,17 +771,19 @@ k_pat_sample(int N, int lda, const double *__restrict__ AL, const double *__rest
 }
 
 // Pattern id of every row: the table row whose seven values equal the
-// row's bit for bit, else PAT_NONE; *nnone counts the latter.  The ids past
-// N (up to a multiple of 4 plus 64) are PAT_NONE.
+// row's bit for bit, else PAT_NONE; cnt[0] counts the latter, cnt[1] the
+// pattern rows whose last two slots are both adjacent rows or ghosts.  The ids
+// past N (up to a multiple of 4 plus 64) are PAT_NONE.
 __global__ void __launch_bounds__(BS)
 k_pat_assign(int N, int npad, int lda, const double *__restrict__ AL, const double *__restrict__ D,
-             const double *__restrict__ tab, int npat, uint8_t *__restrict__ pid, int *__restrict__ nnone) {
+             const int *__restrict__ LL, const double *__restrict__ tab, int npat, uint8_t *__restrict__ pid,
+             int *__restrict__ cnt) {
     __shared__ unsigned long long t[PAT_MAX * PAT_W];
     if (threadIdx.x < PAT_MAX * PAT_W)
         t[threadIdx.x] = threadIdx.x < npat * PAT_W ? (unsigned long long)__double_as_longlong(tab[threadIdx.x]) : 0ull;
     __syncthreads();
     const int i = blockIdx.x * BS + threadIdx.x;
-    int none = 0;
+    int none = 0, adj = 0;
     if (i < N) {
         unsigned long long v[PAT_W];
 #pragma unroll
@@ -796,15 +798,21 @@ k_pat_assign(int N, int npad, int lda, const double *__restrict__ AL, const doub
         }
         pid[i] = (uint8_t)id;
         none = id == PAT_NONE;
+        const int a = LL[4 * (size_t)lda + i], b = LL[5 * (size_t)lda + i];
+        adj = !none && (a > N || abs(a - 1 - i) == 1) && (b > N || abs(b - 1 - i) == 1);
     } else if (i < npad) {
         pid[i] = (uint8_t)PAT_NONE;
     }
-    __shared__ int cnt;
-    if (threadIdx.x == 0) cnt = 0;
+    __shared__ int sum[2];
+    if (threadIdx.x < 2) sum[threadIdx.x] = 0;
     __syncthreads();
-    if (none) atomicAdd(&cnt, 1);
+    const int nn = __popcll(__ballot(none)), na = __popcll(__ballot(adj));
+    if ((threadIdx.x & 63) == 0) {
+        if (nn) atomicAdd(&sum[0], nn);
+        if (na) atomicAdd(&sum[1], na);
+    }
     __syncthreads();
-    if (threadIdx.x == 0 && cnt) atomicAdd(nnone, cnt);
+    if (threadIdx.x < 2 && sum[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], sum[threadIdx.x]);
 }
 
 // FP64 PM stage for an operator with row patterns: k_pm_v2's stage (NT, DOT

@@ -31,6 +31,7 @@
 
 #include "clowns_pcg.h"
 #include "pcg_kernels.hpp"
+#include "run_kernels.hpp"
 #include "assembly_kernels.hpp"
 #include "classify_kernels.hpp"
 #include "vof_kernels.hpp"
@@ -253,6 +254,13 @@ struct Knobs {
     // when a row has its own -- were slower: two inner iterations 1375
     // against 1217 us at 13.1M rows; they keep the coefficient columns.)
     int pm_pat = -1;
+    // Row runs (run_kernels.hpp) for operators with row patterns.  One solve,
+    // off against on: FP64 35.3 against 26.8 ms at 2.45M rows (wavy bed), 263
+    // against 219 at 13.1M (a bathymetry's, 6% of the rows at partial cells);
+    // mixed 27.8 against 23.0 and 159 against 131.5.
+    // CLOWNS_RUNS = 0 off, 1 on wherever there are patterns; -1 (default): from
+    // RUN_MIN_ROWS rows, unless a switch names a form of the kernels they replace.
+    int runs = -1;
     // CLOWNS_VERBOSE = 1: report per-operator tuning decisions on stderr.
     bool verbose = false;
 };
@@ -289,6 +297,26 @@ struct clowns_solver {
     int npat = 0;          // rows in ptab (kept for the next operator)
     int pat_rows = 0;      // rows of the resident operator on a pattern
     bool pat_ok = false;
+    // Row runs (k_run_build), valid if run_ok: a block's tasks in its RUN_TASKS
+    // entries, then packed in the order of launch.
+    DevBuf<int> run_n;            // per block: table tasks, own tasks; scan of both
+    DevBuf<RunPair<double>> run_raw[2], run_pair[2];
+    DevBuf<RunSpmv<double>> run_raws, run_spmv;
+    DevBuf<RunPair<float>> run_pair32[2];
+    DevBuf<RunSpmv<float>> run_spmv32;
+    DevBuf<int4> run_lj;          // lj0, lj1, lj2
+    DevBuf<double> run_c;         // list coefficients
+    DevBuf<float> run_c32;        // the operator's, then the preconditioner's
+    DevBuf<uint8_t> run_cid;
+    DevBuf<int2> run_rq;
+    DevBuf<RunWave> run_wave, run_wave32;
+    DevBuf<int2> run_rj;
+    DevBuf<double> run_rc;
+    DevBuf<float> run_rc32;
+    int run_lcap = 0, run_nl = 0, run_nr = 0, run_nt[2] = {0, 0};
+    bool run_ok = false;
+    bool run_dot = false;         // described for k_pm_dot_run
+    int pat_adj = 0;              // pattern rows whose last two slots are adjacent rows or ghosts
     DevBuf<float> AL32, D32;
     DevBuf<float> ALr32;   // row-major FP32 coefficients of the FP32 SpMV (Knobs::rows32)
     DevBuf<short> Lr16;    // row-major 16-bit codes of the same
@@ -431,6 +459,8 @@ template <typename T> struct Op {
     const uint8_t *pid = nullptr;   // row pattern ids and table (NL = 6), or null
     const double *ptab = nullptr;
     bool pc2 = false;               // FP64 PM stages as k_pm_p2 (with pid; tune_stream)
+    RunOp<T> run = {};              // row runs; spmv null: none
+    RunGrid run_grid = {0, 0, 0};
     KProf *prof = nullptr;          // armed kernel profile, or null
 };
 
@@ -478,10 +508,52 @@ void launch_pm2_c(hipStream_t s, const Scal *sc, const Op<T> &A, const C *AL, in
         launch_pm2_ix<T, C>(s, G2, sc, A, AL + o0, ix32(A, o0), AL + o1, ix32(A, o1), in, out);
 }
 
-// Stages j and j+1 of LDUSUB fused (k_pm2_v2).
+// The two-term stage by k_pm_dot_run; returns the number of its dot partials.
+template <typename T, bool ST, typename C>
+int launch_dot_run_st(hipStream_t s, const Scal *sc, const Op<T> &A, const T *in, T *out, int dot, const T *w,
+                      double *part) {
+    const int G = geo_of(A.N, sizeof(T) == 8 ? 2 : 4).G;
+    auto go = [&](auto kern) { klaunch(kern, G, BS, s, sc, A.N, in, out, w, part, A.run); };
+    switch (dot) {
+    case 0: go(k_pm_dot_run<T, 0, ST, C>); break;
+    case 1: go(k_pm_dot_run<T, 1, ST, C>); break;
+    case 2: go(k_pm_dot_run<T, 2, ST, C>); break;
+    default: go(k_pm_dot_run<T, 3, ST, C>);
+    }
+    return G;
+}
+template <typename T>
+int launch_dot_run(hipStream_t s, const Scal *sc, const Op<T> &A, const T *in, T *out, int dot, const T *w,
+                   double *part) {
+    KScope ks(A.prof, kcls<T>(KC_PMDOT));
+    if constexpr (sizeof(T) == 4) {
+        if (A.ALh)
+            return A.st_pm ? launch_dot_run_st<T, true, _Float16>(s, sc, A, in, out, dot, w, part)
+                           : launch_dot_run_st<T, false, _Float16>(s, sc, A, in, out, dot, w, part);
+    }
+    return A.st_pm ? launch_dot_run_st<T, true, T>(s, sc, A, in, out, dot, w, part)
+                   : launch_dot_run_st<T, false, T>(s, sc, A, in, out, dot, w, part);
+}
+
+// Stages j and j+1 of LDUSUB fused (k_pm2_v2, k_pm_pair_run).
 template <typename T>
 void launch_pm2(hipStream_t s, const Scal *sc, const Op<T> &A, int j, const T *in, T *out) {
     KScope ks(A.prof, kcls<T>(KC_PM2));
+    if (A.run.spmv) {
+        const RunGrid g = A.run_grid;
+        auto go = [&](auto kern) { klaunch(kern, g.own + g.list + g.tab, BS, s, sc, A.N, in, out, A.run, g); };
+        auto form = [&](auto c) {
+            typedef decltype(c) C;
+            if (j == 0)
+                A.st_pm ? go(k_pm_pair_run<T, 0, true, C>) : go(k_pm_pair_run<T, 0, false, C>);
+            else
+                A.st_pm ? go(k_pm_pair_run<T, 1, true, C>) : go(k_pm_pair_run<T, 1, false, C>);
+        };
+        if constexpr (sizeof(T) == 4) {
+            if (A.ALh) return form(_Float16());
+        }
+        return form(T());
+    }
     if constexpr (sizeof(T) == 4) {
         if (A.ALh) {
             launch_pm2_c<T, _Float16>(s, sc, A, A.ALh, j, in, out);
@@ -595,11 +667,12 @@ int launch_pm_stage(hipStream_t s, const Scal *sc, const Op<T> &A, int j, const 
 template <typename T>
 int apply_pm(hipStream_t s, const Scal *sc, const Op<T> &A, const T *in, T *out, T *y, T *t, int dot, const T *w,
              double *part) {
-    if (A.fuse) {
+    if (A.fuse || A.run.spmv) {
         // stages (1,2) and (3,4) fused pairwise; 5/6 (two-term) carries the dots
         launch_pm2<T>(s, sc, A, 0, in, t);
         if (A.NL == 6) {
             launch_pm2<T>(s, sc, A, 2, t, y);
+            if (A.run.cid) return launch_dot_run<T>(s, sc, A, y, out, dot, w, part);
             return launch_pm_stage<T, 2>(s, sc, A, 4, y, out, dot, w, part);
         }
         // NL = 4: stage 3 alone, then stage 4 with the dots
@@ -751,6 +824,18 @@ void launch_spmv_v2(hipStream_t s, const Scal *sc, const Op<T> &A, IX ix, int mo
 template <typename T>
 void spmv(hipStream_t s, const Scal *sc, const Op<T> &A, int mode, const T *x, const T *v1, T *y) {
     KScope ks(A.prof, kcls<T>(mode == 3 ? KC_RESID : KC_SPMV));
+    if (A.run.spmv) {
+        const RunGrid g = A.run_grid;
+        auto go = [&](auto kern) { klaunch(kern, g.own + g.list + g.tab, BS, s, sc, A.N, x, v1, y, A.run, g); };
+        if constexpr (sizeof(T) == 8) {  // the true residual is FP64 only
+            if (mode == 3) {
+                go(k_spmv_run<T, 3>);
+                return;
+            }
+        }
+        go(k_spmv_run<T, 0>);
+        return;
+    }
     if (A.NL == 6) {
         if (has8(A))
             launch_spmv_v2<T, 6, Ix8>(s, sc, A, ix8(A, 0), mode, x, v1, y);
@@ -907,7 +992,7 @@ template <typename T> void tune_stream(clowns_solver *h, Op<T> &A, VecSet<T> &V)
 // forms the solver runs).
 template <typename T> void known_stream(const clowns_solver *h, Op<T> &A) {
     int f;
-    if (stored_forms(h, A, &f)) set_forms(A, f);
+    if (!A.run.spmv && stored_forms(h, A, &f)) set_forms(A, f);
 }
 
 // How many iterations to enqueue next.  The device decides convergence
@@ -1037,9 +1122,10 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
 
 int check_nl(int NL) { return (NL == 6 || NL == 4) ? CLOWNS_OK : CLOWNS_EBADNL; }
 
-int build_ll16(clowns_solver *h);
 int build_ll8(clowns_solver *h);
-int build_patterns(clowns_solver *h);
+int build_forms(clowns_solver *h);
+int build_runs32(clowns_solver *h);
+int order_runs(clowns_solver *h);
 int ensure_block_order(clowns_solver *h);
 
 // Load AL/LL/D (reference layout, stride lda) from `kind` memory and scale +
@@ -1296,7 +1382,7 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     const int ldu = lda;
     lda = (N + 63) & ~63;
     const size_t nm = (size_t)lda * NL;
-    if ((rc = h->AL.ensure(nm)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure(N)) ||
+    if ((rc = h->AL.ensure(nm + RUN_PAD)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure((size_t)N + RUN_PAD)) ||
         (rc = h->W.ensure(N)))
         return rc;
     if ((rc = ensure_common(h, N))) return rc;
@@ -1350,15 +1436,14 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     h->will_rev_valid = false;
     h->order_G = 0;  // a caller's operator: natural order unless set_block_order
     h->order_pending = false;
-    int rc2 = build_ll16(h);
-    return rc2 ? rc2 : build_patterns(h);
+    return build_forms(h);
 }
 
 int ensure_f32(clowns_solver *h) {
     if (h->have32) return CLOWNS_OK;
     int rc;
     const size_t nm = (size_t)h->lda * h->NL;
-    if ((rc = h->AL32.ensure(nm)) || (rc = h->D32.ensure(h->N))) return rc;
+    if ((rc = h->AL32.ensure(nm + RUN_PAD)) || (rc = h->D32.ensure((size_t)h->N + RUN_PAD))) return rc;
     hipStream_t s = h->stream;
     k_to_f32<<<cdiv(h->N, BS), BS, 0, s>>>(h->N, h->lda, h->NL, h->AL.p, h->D.p, h->AL32.p, h->D32.p);
     if (h->kn.pm_half) {
@@ -1367,7 +1452,8 @@ int ensure_f32(clowns_solver *h) {
     }
     h->have_h = h->kn.pm_half;
     h->have_rows = h->have_rows8 = false;
-    if (h->kn.rows32 && h->NL == 6 && h->ll16_ok) {
+    if ((rc = build_runs32(h))) return rc;
+    if (h->kn.rows32 && h->NL == 6 && h->ll16_ok && !h->run_ok) {
         const size_t n6 = (size_t)6 * h->N;
         if ((rc = h->ALr32.ensure(n6)) || (rc = h->Lr16.ensure(n6)) || (rc = h->nonunit.ensure(1))) return rc;
         if (h->ll8_ok && (rc = h->Lr8.ensure(n6))) return rc;
@@ -1448,13 +1534,16 @@ constexpr int PAT_SAMPLE = 1 << 15;
 int assign_patterns(clowns_solver *h, int *nnone) {
     hipStream_t s = h->stream;
     const int N = h->N;
-    fill<int>(s, h->flag.p, 1, 0);
+    fill<int>(s, h->flag.p, 2, 0);
     const int npad = n_pad(N) + 4;
-    k_pat_assign<<<cdiv(npad, BS), BS, 0, s>>>(N, npad, h->lda, h->AL.p, h->D.p, h->ptab.p, h->npat, h->pid.p,
-                                               h->flag.p);
+    k_pat_assign<<<cdiv(npad, BS), BS, 0, s>>>(N, npad, h->lda, h->AL.p, h->D.p, h->LL.p, h->ptab.p, h->npat,
+                                               h->pid.p, h->flag.p);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(nnone, h->flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    int res[2] = {0, 0};
+    HIPCHK(hipMemcpyAsync(res, h->flag.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
+    *nnone = res[0];
+    h->pat_adj = res[1];
     return CLOWNS_OK;
 }
 
@@ -1465,7 +1554,7 @@ int build_patterns(clowns_solver *h) {
     if (!h->kn.patterns || h->NL != 6 || N < PAT_MIN_ROWS) return CLOWNS_OK;
     int rc;
     if ((rc = h->pid.ensure((size_t)n_pad(N) + 4)) || (rc = h->ptab.ensure(PAT_MAX * PAT_W)) ||
-        (rc = h->flag.ensure(1)))
+        (rc = h->flag.ensure(2)))
         return rc;
     hipStream_t s = h->stream;
     int nnone = N;
@@ -1510,6 +1599,173 @@ int build_patterns(clowns_solver *h) {
     return CLOWNS_OK;
 }
 
+// The packed tasks of one precision in a block order (null: natural).
+template <typename T, typename C>
+int pack_runs(clowns_solver *h, const int *order, DevBuf<RunPair<T>> *pair, DevBuf<RunSpmv<T>> &sp,
+              DevBuf<RunWave> &wave) {
+    const int nblk = cdiv(h->N, RUN_ROWS), G = geo_of(h->N, 2).G;
+    constexpr int R = sizeof(T) == 8 ? 2 : 4;
+    const size_t nt = std::max(1, h->run_nt[0] + h->run_nt[1]);
+    const int nw = 4 * geo_of(h->N, R).G;
+    int rc;
+    if ((rc = wave.ensure(nw)) || (rc = pair[0].ensure(nt)) || (rc = pair[1].ensure(nt)) || (rc = sp.ensure(nt))) return rc;
+    hipStream_t s = h->stream;
+    const int *n0 = h->run_n.p, *n1 = n0 + nblk;
+    int *pos = h->run_n.p + 2 * nblk;
+    k_run_counts<<<cdiv(G, BS), BS, 0, s>>>(G, nblk, order, n0, n1, pos);
+    k_cls_scan_blocks<<<1, 1024, 0, s>>>(G, pos);
+    k_cls_scan_blocks<<<1, 1024, 0, s>>>(G, pos + G + 1);
+    k_run_pack<T, C><<<cdiv((long)G * RUN_TASKS, BS), BS, 0, s>>>(G, nblk, order, n0, n1, pos, h->run_raw[0].p,
+                                                                 h->run_raw[1].p, h->run_raws.p, pair[0].p,
+                                                                 pair[1].p, sp.p);
+    if (h->run_dot) k_run_waves<R><<<cdiv(nw, BS), BS, 0, s>>>(nw, nblk, order, h->run_rq.p, wave.p);
+    HIPCHK(hipGetLastError());
+    return CLOWNS_OK;
+}
+
+// Row runs from this size on (below, a solve is bound by its launches and the
+// column kernels' shorter chains of loads win: FP64 solves to 1e-8, columns
+// against runs, 6.6/6.7 ms at 0.46M rows, 9.3/9.4 at 0.72M, 10.2/9.6 at 1.04M,
+// 15.6/13.0 at 1.65M; mixed 11.3/11.5 at 0.72M, 13.9/13.1 at 1.2M).
+constexpr int RUN_MIN_ROWS = 3 << 18;
+
+// The row runs of the resident operator (with row patterns): used while the
+// lists hold at most an eighth of the rows (a listed row costs about as much
+// as 15 in tasks: at 13.1M rows 3% listed are 28 of the SpMV's 88 us, which
+// the column kernel takes 105 for); the two-term form when 9 in 10 pattern
+// rows' last two slots are the adjacent rows or ghosts and at most an eighth
+// of the rows need a record.
+int build_runs(clowns_solver *h) {
+    h->run_ok = h->run_dot = false;
+    if (!h->pat_ok || h->kn.runs == 0 || (h->kn.runs < 0 && h->N < RUN_MIN_ROWS) || h->N > RUN_MAX_N) return CLOWNS_OK;
+    const int N = h->N, nblk = cdiv(N, RUN_ROWS), G = geo_of(N, 2).G;
+    const size_t nt = (size_t)nblk * RUN_TASKS;
+    const bool dot = h->pat_adj >= h->pat_rows - h->pat_rows / 10;
+    const int lcap = N / 8, rcap = dot ? N / 8 : 1;
+    int rc;
+    if ((rc = h->run_n.ensure(2 * (size_t)nblk + 2 * (size_t)(G + 1))) || (rc = h->run_raw[0].ensure(nt)) ||
+        (rc = h->run_raw[1].ensure(nt)) || (rc = h->run_raws.ensure(nt)) ||
+        (rc = h->run_lj.ensure(3 * (size_t)lcap)) || (rc = h->run_c.ensure(RUN_LC * (size_t)lcap)) ||
+        (rc = h->flag.ensure(4)))
+        return rc;
+    if (dot && ((rc = h->run_cid.ensure((size_t)nblk * RUN_ROWS)) || (rc = h->run_rq.ensure(4 * (size_t)nblk)) ||
+                (rc = h->run_rj.ensure(rcap)) || (rc = h->run_rc.ensure(2 * (size_t)rcap))))
+        return rc;
+    hipStream_t s = h->stream;
+    fill<int>(s, h->flag.p, 4, 0);
+    RunBuild o;
+    o.nt0 = h->run_n.p;
+    o.nt1 = o.nt0 + nblk;
+    o.pair0 = h->run_raw[0].p;
+    o.pair1 = h->run_raw[1].p;
+    o.spmv = h->run_raws.p;
+    o.lj0 = h->run_lj.p;
+    o.lj1 = o.lj0 + lcap;
+    o.lj2 = reinterpret_cast<int2 *>(o.lj1 + lcap);
+    o.lc = h->run_c.p;
+    o.cid = dot ? h->run_cid.p : nullptr;
+    o.rq = h->run_rq.p;
+    o.rj = h->run_rj.p;
+    o.rc = h->run_rc.p;
+    o.lcap = lcap;
+    o.rcap = rcap;
+    k_run_build<<<nblk, BS, 0, s>>>(N, h->lda, h->AL.p, h->D.p, h->LL.p, h->pid.p, o, h->flag.p);
+    HIPCHK(hipGetLastError());
+    int res[4] = {0, 0, 0, 0};
+    HIPCHK(hipMemcpyAsync(res, h->flag.p, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    h->run_lcap = lcap;
+    h->run_nl = res[0];
+    h->run_nr = res[1];
+    h->run_nt[0] = res[2];
+    h->run_nt[1] = res[3];
+    if (h->kn.verbose)
+        fprintf(stderr, "clowns_pcg: N=%d row runs: %d tasks, %d with their own coefficients, %d rows listed, "
+                        "%d records\n", N, res[2], res[3], res[0], res[1]);
+    if (res[0] > lcap) return CLOWNS_OK;
+    h->run_ok = true;
+    h->run_dot = dot && res[1] <= rcap;
+    return pack_runs<double, double>(h, nullptr, h->run_pair, h->run_spmv, h->run_wave);
+}
+// What the kernels read of the resident operator beside its columns: the row
+// patterns, then the row runs, or the index codes of the column kernels.
+int build_forms(clowns_solver *h) {
+    int rc;
+    if ((rc = build_patterns(h)) || (rc = build_runs(h))) return rc;
+    h->ll16_ok = h->ll8_ok = false;
+    h->ll16_wide = h->ll8_wide = 0;
+    return h->run_ok && h->run_dot ? CLOWNS_OK : build_ll16(h);
+}
+// The FP32 forms (ensure_f32).
+int build_runs32(clowns_solver *h) {
+    if (!h->run_ok) return CLOWNS_OK;
+    const size_t nlc = RUN_LC * (size_t)h->run_lcap, nr = h->run_dot ? h->run_nr : 0;
+    int rc;
+    if ((rc = h->run_c32.ensure(2 * nlc)) || (rc = h->run_rc32.ensure(2 * nr + 1)) ||
+        (rc = h->kn.pm_half ? pack_runs<float, _Float16>(h, nullptr, h->run_pair32, h->run_spmv32, h->run_wave32)
+                            : pack_runs<float, float>(h, nullptr, h->run_pair32, h->run_spmv32, h->run_wave32)))
+        return rc;
+    hipStream_t s = h->stream;
+    auto list = [&](auto kern, int n, int W, int cap, const double *a, float *b) {
+        if (n) kern<<<cdiv(n, BS), BS, 0, s>>>(n, W, cap, a, b);
+    };
+    list(k_run_list32<float>, h->run_nl, RUN_LC, h->run_lcap, h->run_c.p, h->run_c32.p);
+    auto pm = [&](auto kern) {
+        list(kern, h->run_nl, RUN_LC, h->run_lcap, h->run_c.p, h->run_c32.p + nlc);
+        list(kern, 2 * nr, 1, 0, h->run_rc.p, h->run_rc32.p);
+    };
+    h->kn.pm_half ? pm(k_run_list32<_Float16>) : pm(k_run_list32<float>);
+    HIPCHK(hipGetLastError());
+    return CLOWNS_OK;
+}
+// The FP64 tasks in the operator's block order, once it is known (order_G set).
+int order_runs(clowns_solver *h) {
+    if (!h->run_ok || h->order_G != geo_of(h->N, 2).G) return CLOWNS_OK;
+    return pack_runs<double, double>(h, h->order.p, h->run_pair, h->run_spmv, h->run_wave);
+}
+template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
+    if (!h->run_ok) return;
+    RunOp<T> &d = A.run;
+    const size_t lcap = h->run_lcap;
+    if constexpr (sizeof(T) == 8) {
+        d.pair[0] = h->run_pair[0].p;
+        d.pair[1] = h->run_pair[1].p;
+        d.spmv = h->run_spmv.p;
+        d.sc = d.lc = h->run_c.p;
+        d.rc = h->run_rc.p;
+    } else {
+        if (!h->have32) return;
+        d.pair[0] = h->run_pair32[0].p;
+        d.pair[1] = h->run_pair32[1].p;
+        d.spmv = h->run_spmv32.p;
+        d.sc = h->run_c32.p;
+        d.lc = d.sc + RUN_LC * lcap;
+        d.rc = h->run_rc32.p;
+    }
+    d.lj0 = h->run_lj.p;
+    d.lj1 = d.lj0 + lcap;
+    d.lj2 = reinterpret_cast<const int2 *>(d.lj1 + lcap);
+    d.AL = A.AL;
+    d.D = A.D;
+    d.cid = h->run_dot ? h->run_cid.p : nullptr;
+    d.wave = sizeof(T) == 8 ? h->run_wave.p : h->run_wave32.p;
+    d.rj = h->run_rj.p;
+    d.ptab = h->ptab.p;
+    d.lda = h->lda;
+    d.lcap = h->run_lcap;
+    d.nl = h->run_nl;
+    d.nt[0] = h->run_nt[0];
+    d.nt[1] = h->run_nt[1];
+    A.run_grid = {cdiv(d.nt[1], 4 * RUN_U), cdiv(d.nl, BS), (cdiv(d.nt[0], 4 * RUN_U) + 7) & ~7};
+    // Streamed PM stages where the three vectors of the stage with dots
+    // outgrow three quarters of the 256 MB last-level cache (cached against
+    // streamed, ms a solve to 1e-8; FP64 wavy bed: 74.4/74.0 at 9.8M rows,
+    // 110.2/107.9 at 12.2M, 449/436 at 24.3M, but 41.7/42.0 at 7.4M; FP32:
+    // 157.5/156.3 at 19.5M, 240/232 at 30.4M, but 131.5/134.4 at 13.1M).  The
+    // SpMV gained nothing from it (88.2 against 88.4 us at 13.1M).
+    A.st_pm = (size_t)h->N * 3 * sizeof(T) > ((size_t)192 << 20);
+}
+
 // Views of the resident operator.
 Op<double> op64(const clowns_solver *h) {
     Op<double> A{h->N, h->NL, h->lda, h->AL.p, h->LL.p, h->D.p};
@@ -1526,6 +1782,7 @@ Op<double> op64(const clowns_solver *h) {
         A.pid = h->pid.p;
         A.ptab = h->ptab.p;
     }
+    use_runs(h, A);
     return A;
 }
 Op<float> op32(const clowns_solver *h) {
@@ -1558,6 +1815,7 @@ Op<float> op32(const clowns_solver *h) {
             A.base8 = nullptr;
         }
     }
+    use_runs(h, A);
     return A;
 }
 
@@ -1570,13 +1828,15 @@ Op<float> op32(const clowns_solver *h) {
 // neighbours with one 8-byte load (k_spmv_rows32), which through the last
 // ghost row reads the entry after it (its value is not used: the second row
 // of that pair has another neighbour and loads it on its own).
+// The row-run kernels read up to RUN_PAD zero rows.
 constexpr int VEC_SLACK = 4;
+constexpr int VEC_PAD = std::max(PAD + VEC_SLACK, RUN_PAD);
 template <typename T> int ensure_vecs(clowns_solver *h, VecSet<T> &V, int N) {
-    int rc = V.ensure((size_t)n_pad(N) + VEC_SLACK);
+    int rc = V.ensure((size_t)N + VEC_PAD);
     if (rc) return rc;
     if (V.padN != N) {
         T *all[] = {V.r.p, V.rh.p, V.p0.p, V.q.p, V.e.p, V.v.p, V.y.p, V.t.p, V.x.p};
-        for (T *b : all) fill<T>(h->stream, b + N, PAD, T(0));
+        for (T *b : all) fill<T>(h->stream, b + N, VEC_PAD, T(0));
         V.padN = N;
     }
     return CLOWNS_OK;
@@ -1585,10 +1845,10 @@ template <typename T> int ensure_vecs(clowns_solver *h, VecSet<T> &V, int N) {
 // The scaled right-hand side of a run (the mixed solve gathers it in its
 // first PM application): N + 64 entries, ghost rows zero.
 int ensure_bs(clowns_solver *h, int N) {
-    int rc = h->bs.ensure((size_t)n_pad(N));
+    int rc = h->bs.ensure((size_t)N + VEC_PAD);
     if (rc) return rc;
     if (h->bs_padN != N) {
-        fill<double>(h->stream, h->bs.p + N, PAD, 0.0);
+        fill<double>(h->stream, h->bs.p + N, VEC_PAD, 0.0);
         h->bs_padN = N;
     }
     return CLOWNS_OK;
@@ -1605,8 +1865,10 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
     VecSet<double> &V = h->v64;
     if ((rc = ensure_vecs(h, V, A_in.N)) || (rc = ensure_bs(h, A_in.N))) return rc;
     Op<double> A = A_in;
-    A.fuse = tune_fuse(h, A, V);
-    tune_stream(h, A, V);
+    if (!A.run.spmv) {
+        A.fuse = tune_fuse(h, A, V);
+        tune_stream(h, A, V);
+    }
     if (h->prof.on) A.prof = &h->prof;
     const int N = A.N;
     const int G1 = geo_of(N, 1).G;
@@ -1663,10 +1925,12 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
         return rc;
     Op<double> A = A_in;
     Op<float> A32 = A32_in;
-    A.fuse = tune_fuse(h, A, V);
-    A32.fuse = tune_fuse(h, A32, F);
-    tune_stream(h, A, V);
-    tune_stream(h, A32, F);
+    if (!A.run.spmv) {
+        A.fuse = tune_fuse(h, A, V);
+        A32.fuse = tune_fuse(h, A32, F);
+        tune_stream(h, A, V);
+        tune_stream(h, A32, F);
+    }
     if (h->prof.on) A.prof = A32.prof = &h->prof;
     const int N = A.N;
     const int G1 = geo_of(N, 1).G;
@@ -1816,6 +2080,11 @@ extern "C" int clowns_solver_create(clowns_solver **out, int device, void *strea
         flag("CLOWNS_BLOCK_ORDER", k.block_order);
         flag("CLOWNS_VERBOSE", k.verbose);
         flag("CLOWNS_PATTERNS", k.patterns);
+        tri("CLOWNS_RUNS", k.runs);
+        if (k.runs < 0)
+            for (const char *name : {"CLOWNS_FUSE_PM", "CLOWNS_STREAM", "CLOWNS_LL8", "CLOWNS_PM_PAT", "CLOWNS_LL16",
+                                     "CLOWNS_V4_32", "CLOWNS_SPMV_ROWS", "CLOWNS_SPMV32_P2"})
+                if (getenv(name)) k.runs = 0;
         flag("CLOWNS_CLASSIFY_HOST", h->cls_force_host);
         if (const char *e = getenv("CLOWNS_POLL")) h->poll = std::max(1, atoi(e));
         if (const char *e = getenv("CLOWNS_TAU_MIN")) h->tau_min = std::max(1e-8, atof(e));
@@ -1830,7 +2099,9 @@ extern "C" int clowns_solver_destroy(clowns_solver *h) {
     (void)hipSetDevice(h->device);
     (void)hipStreamSynchronize(h->stream);
     h->AL.release(); h->D.release(); h->W.release(); h->LL.release(); h->LL16.release(); h->base16.release(); h->LL8.release(); h->base8.release(); h->order.release(); h->order_first.release();
-    h->AL32.release(); h->D32.release(); h->ALh.release(); h->ALr32.release(); h->Lr16.release(); h->Lr8.release(); h->nonunit.release(); h->pid.release(); h->ptab.release(); h->pat_keys.release();
+    h->AL32.release(); h->D32.release(); h->ALh.release(); h->ALr32.release(); h->Lr16.release(); h->Lr8.release(); h->nonunit.release(); h->pid.release(); h->ptab.release();
+    h->run_n.release(); h->run_raw[0].release(); h->run_raw[1].release(); h->run_raws.release(); h->run_pair[0].release(); h->run_pair[1].release(); h->run_spmv.release(); h->run_pair32[0].release(); h->run_pair32[1].release(); h->run_spmv32.release(); h->run_lj.release(); h->run_c.release(); h->run_c32.release(); h->run_cid.release(); h->run_rq.release(); h->run_wave.release(); h->run_wave32.release(); h->run_rj.release(); h->run_rc.release(); h->run_rc32.release();
+    h->pat_keys.release();
     h->ALt.release(); h->Dt.release(); h->Wt.release(); h->LLt.release();
     h->LLt16.release(); h->baset16.release(); h->LLt8.release(); h->baset8.release();
     h->AL0.release(); h->D0.release(); h->LL0.release();
@@ -1891,13 +2162,14 @@ extern "C" int clowns_solver_solve(clowns_solver *h, const double *d_b, double *
 // their slack, each 256-byte aligned), the scaled right-hand side, the dot
 // partials and the run scalars, for up to NOALLOC_MAX_ROWS rows: 58 MiB.
 constexpr int NOALLOC_MAX_ROWS = 1 << 19;
-constexpr size_t NA_VEC = (size_t)NOALLOC_MAX_ROWS + PAD + 64;             // entries per vector
+constexpr size_t NA_VEC = (size_t)NOALLOC_MAX_ROWS + 704;                  // entries per vector
 constexpr size_t NA_G1 = (((size_t)NOALLOC_MAX_ROWS + BS - 1) / BS + 7) / 8 * 8;  // largest grid
 constexpr size_t NA_V64 = 0;                                                 // 9 FP64 vectors + bs
 constexpr size_t NA_V32 = NA_V64 + 10 * NA_VEC * sizeof(double);             // 9 FP32 vectors
 constexpr size_t NA_PART = NA_V32 + 9 * NA_VEC * sizeof(float);              // 2 x NA_G1 partials
 constexpr size_t NA_SC = NA_PART + 2 * NA_G1 * sizeof(double);               // 2 run scalars
 constexpr size_t NA_BYTES = NA_SC + 2 * sizeof(Scal);
+static_assert(NA_VEC >= (size_t)NOALLOC_MAX_ROWS + VEC_PAD, "room for the zero rows");
 static_assert(NA_VEC * sizeof(float) % 256 == 0 && NA_V32 % 256 == 0 && NA_PART % 256 == 0 && NA_SC % 256 == 0,
               "vectors start 256-byte aligned");
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
@@ -2607,7 +2879,7 @@ int ensure_block_order(clowns_solver *h) {
     HIPCHK(hipMemcpyAsync(h->order.p, ord.data(), (size_t)G * sizeof(int), hipMemcpyHostToDevice, s));
     HIPCHK(hipStreamSynchronize(s));
     h->order_G = G;
-    return CLOWNS_OK;
+    return order_runs(h);
 }
 } // namespace
 
@@ -2619,7 +2891,7 @@ extern "C" int clowns_solver_assemble(clowns_solver *h, const clowns_grid_dev *g
     const int N = g->nrows;
     const int lda = (N + 63) & ~63;
     const size_t nm = (size_t)lda * 6;
-    if ((rc = h->AL.ensure(nm)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure(N)) ||
+    if ((rc = h->AL.ensure(nm + RUN_PAD)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure((size_t)N + RUN_PAD)) ||
         (rc = h->W.ensure(N)))
         return rc;
     if (keep_raw && ((rc = h->AL0.ensure(nm)) || (rc = h->LL0.ensure(nm)) || (rc = h->D0.ensure(N))))
@@ -2642,8 +2914,7 @@ extern "C" int clowns_solver_assemble(clowns_solver *h, const clowns_grid_dev *g
     h->have_t = false;
     h->raw_valid = keep_raw != 0;
     h->will_rev_valid = false;
-    if ((rc = build_ll16(h))) return rc;
-    if ((rc = build_patterns(h))) return rc;
+    if ((rc = build_forms(h))) return rc;
     if ((rc = note_block_order(h, g))) return rc;
     HIPCHK(hipStreamSynchronize(s));
     return CLOWNS_OK;
@@ -3007,6 +3278,14 @@ extern "C" int clowns_solver_tuning(clowns_solver *h, int32_t out[8]) {
     const int fz = h->kn.fuse_pm;
     out[0] = fz >= 0 ? fz : (tuned_size(N, h->fuse64_N) ? h->fuse64 : -1);
     out[1] = fz >= 0 ? fz : (tuned_size(N, h->fuse32_N) ? h->fuse32 : -1);
+    if (h->run_ok) {  // row runs: nothing is timed
+        out[0] = out[1] = out[6] = 1;
+        out[2] = op64(h).st_pm;
+        out[3] = h->have32 ? (int)op32(h).st_pm : -1;
+        out[4] = out[5] = 0;
+        out[7] = h->have32 ? 8 : -1;
+        return CLOWNS_OK;
+    }
     int f[2] = {-1, -1};
     if (!stored_forms(h, op64(h), &f[0])) f[0] = -1;
     if (!stored_forms(h, op32(h), &f[1])) f[1] = -1;
@@ -3042,7 +3321,7 @@ extern "C" int clowns_solver_set_block_order(clowns_solver *h, const int32_t *d_
     if ((rc = h->order.ensure(G))) return rc;
     HIPCHK(hipMemcpy(h->order.p, ho.data(), (size_t)G * sizeof(int), hipMemcpyHostToDevice));
     h->order_G = G;
-    return CLOWNS_OK;
+    return order_runs(h);
 }
 
 extern "C" int clowns_solver_patterns(clowns_solver *h, int32_t *npat, int32_t *rows) {
@@ -3055,6 +3334,7 @@ extern "C" int clowns_solver_patterns(clowns_solver *h, int32_t *npat, int32_t *
 extern "C" int clowns_solver_index_bits(clowns_solver *h) {
     if (!h || h->N < 1) return -CLOWNS_EBADARG;
     int f;
+    if (h->run_ok) return 0;
     if (h->ll8_ok && (h->kn.ll8 == 1 || (stored_forms(h, op64(h), &f) && (f & 4)))) return 8;
     return h->ll16_ok ? 16 : 32;
 }

@@ -612,6 +612,14 @@ CLASS_BYTES = {"spmv": 72, "pm_stage": 24, "pm_pair": 32, "pm_dot": 40, "p_updat
 
 def kernel_names(tune, precision):
     """Names of the kernel forms the solver runs on this operator, per class."""
+    if tune["index64" if precision == "fp64" else "index32"] == 0:  # row runs
+        T, c = ("double", "double") if precision == "fp64" else (
+            "float", "_Float16" if os.environ.get("CLOWNS_PM_HALF", "1") != "0" else "float")
+        st = "true" if tune["stream64" if precision == "fp64" else "stream32"] == 1 else "false"
+        V = "vec<%s>" % T
+        return {"spmv": f"k_spmv_run<{T},0>", "pm_pair": f"k_pm_pair_run<{T},S,{st},{c}>",
+                "pm_dot": f"k_pm_dot_run<{T},DOT,{st},{c}>", "p_update": "k_pupd_" + V, "e_update": "k_eupd_" + V,
+                "xr_update": "k_update_" + V, "residual_spmv": f"k_spmv_run<{T},3>"}
     if precision == "fp64":
         st = tune["stream64"]
         pm, sp = ("true" if st > 0 and st & 1 else "false"), ("true" if st > 0 and st & 2 else "false")

@@ -457,12 +457,13 @@ int clowns_solver_vof_time_kernel(clowns_solver *h, const clowns_grid_dev *g,
  * stages (FP64, FP32: 1 fused, 0 single); out[2], out[3] streamed
  * (non-temporal) arrays (FP64, FP32: bit 0 the PM stages, bit 1 the SpMV);
  * out[4], out[5] the width of the neighbour-index codes (FP64, FP32: 8, 16
- * or 32); out[6] 1 if the FP64 PM stages read pattern rows' coefficients
- * from the row-pattern table (two 128-row chunks a wavefront), else 0;
- * out[7] the FP32 SpMV's form: 0 column-major, 1 row-major copies, 2
- * row-major in two 128-row chunks a wavefront, plus 4 when it
- * reads pattern rows' coefficients from the row-pattern table.  -1 where
- * not yet decided.  No counterpart in the reference (reporting). */
+ * or 32; 0: the operator runs by row runs, whose descriptions stand in for
+ * codes); out[6] 1 if the FP64 PM stages read pattern rows' coefficients
+ * from the row-pattern table or from row runs, else 0; out[7] the FP32
+ * SpMV's form: 0 column-major, 1 row-major copies, 2 row-major in two
+ * 128-row chunks a wavefront, plus 4 when it reads pattern rows'
+ * coefficients from the row-pattern table, or 8 for row runs.  -1 where not
+ * yet decided.  No counterpart in the reference (reporting). */
 int clowns_solver_tuning(clowns_solver *h, int32_t out[8]);
 
 /* Run the resident operator's gather kernels (SpMV, PM stages) over their
@@ -481,7 +482,8 @@ int clowns_solver_set_block_order(clowns_solver *h, const int32_t *d_order, int3
  * classes with 6-bit steps; the few slots that do not fit read the 32-bit
  * LL; chosen per operator when it is first solved, or forced), 16 for the
  * 16-bit codes (every offset fits; always for box grids of up to 16383
- * cells a line), else 32; negative CLOWNS_E* on error.  No counterpart in
+ * cells a line), else 32; 0 where it runs by row runs, which read none;
+ * negative CLOWNS_E* on error.  No counterpart in
  * the reference (diagnostics). */
 int clowns_solver_index_bits(clowns_solver *h);
 
