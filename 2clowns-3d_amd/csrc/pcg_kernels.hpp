@@ -52,6 +52,16 @@ struct Scal {
     int pad_[2];
 };
 
+// The word the host polls: iterations done and whether the run ended, above
+// ERR in single precision.
+__device__ __forceinline__ unsigned long long run_word(int K, int done, double err) {
+    return (unsigned long long)(unsigned)(2 * K + (done ? 1 : 0)) << 32 | (unsigned)__float_as_int((float)err);
+}
+__device__ __forceinline__ void post_word(unsigned long long *host, int K, int done, double err) {
+    if (host)
+        __hip_atomic_store(host, run_word(K, done, err), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own
 // L2.  Giving XCD x the contiguous logical blocks [x*G/8, (x+1)*G/8) keeps the
 // +-1, +-row and +-plane neighbours of a row in the L2 that streamed them.
@@ -1567,7 +1577,8 @@ k_update_vec(const Scal *__restrict__ sc, int N, T *__restrict__ x, const T *__r
 template <typename T>
 __global__ void __launch_bounds__(BS)
 k_pupd_vec(const Scal *__restrict__ sc, int N, T *__restrict__ p, const T *__restrict__ r,
-           const T *__restrict__ q) {
+           const T *__restrict__ q, unsigned long long *host) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) post_word(host, sc->K, sc->done, sc->ERR);
     if (sc->done) return;
     using VT = typename VecOf<T>::t;
     constexpr int RV = VecOf<T>::R;
@@ -1662,7 +1673,7 @@ __global__ void k_reset(Scal *sc, double eps, int itermax, int beta_prod) {
 // After k_init: BN, C1.  A zero right-hand side with a zero residual returns
 // at once with X unchanged (the reference divides 0/0 there).
 __global__ void __launch_bounds__(FIN_BS)
-k_fin_init(Scal *sc, const double *__restrict__ part, int G) {
+k_fin_init(Scal *sc, const double *__restrict__ part, int G, unsigned long long *host) {
     if (sc->done) return;
     double r[2];
     fin_sums<2>(part, G, r);
@@ -1677,6 +1688,7 @@ k_fin_init(Scal *sc, const double *__restrict__ part, int G) {
             sc->kout = 0;
             sc->ier = 0;
             sc->done = 1;
+            post_word(host, 0, 1, 0.0);
         }
     }
 }
@@ -1706,49 +1718,54 @@ k_fin_omega(Scal *sc, const double *__restrict__ part, int G) {
     }
 }
 
-// ERR and the exits in the reference's order (pcgpme_para.F90:215-251).
-__global__ void __launch_bounds__(FIN_BS)
-k_fin_beta(Scal *sc, const double *__restrict__ part, int G, int K) {
-    if (sc->done) return;
-    const double BN = sc->BN, ERRP = sc->ERRP, EPS = sc->EPS, AMU = sc->AMU, RQ = sc->RQ;
-    const int beta_prod = sc->beta_prod, itermax = sc->itermax;
-    double r[2];
-    fin_sums<2>(part, G, r);
-    const double rn = r[0], c1 = r[1];
-    if (threadIdx.x != 0) return;
-    sc->RN = rn;
-    sc->C1 = c1;
-    sc->K = K;
-    const double err = sqrt(rn / BN);
-    sc->ERR = err;
+// ERR and the exits in the reference's order (pcgpme_para.F90:215-251), after
+// iteration s.K + 1.
+__device__ __forceinline__ void beta_step(Scal &s, double rn, double c1) {
+    const int K = s.K + 1;
+    s.RN = rn;
+    s.C1 = c1;
+    s.K = K;
+    const double err = sqrt(rn / s.BN);
+    s.ERR = err;
     int stop = 0;
     if (!(err == err) || err > 1.7976931348623157e308) {
-        sc->ier = 4001; // CLOWNS_ENONFINITE
+        s.ier = 4001;  // CLOWNS_ENONFINITE
         stop = 1;
-    } else if (K >= 10 && fabs(err - ERRP) <= err * 1.0e-6) {
+    } else if (K >= 10 && fabs(err - s.ERRP) <= err * 1.0e-6) {
         stop = 1;
-    } else if (err <= EPS) {
+    } else if (err <= s.EPS) {
         stop = 1;
     } else {
-        sc->ERRP = err;
-        if (AMU == 0.0 || c1 == 0.0) {
+        s.ERRP = err;
+        if (s.AMU == 0.0 || c1 == 0.0) {
             stop = 1;
         } else {
             // Same quantity, two roundings: pcgpme_para.F90:241 divides
             // twice, pcgpme_2DH.f90:241 divides by the product.
-            sc->BETA = beta_prod ? c1 / (AMU * RQ) : c1 / AMU / RQ;
-            if (K >= itermax) {
-                sc->ier = 3000;
-                sc->kout = K + 1;
-                sc->done = 1;
+            s.BETA = s.beta_prod ? c1 / (s.AMU * s.RQ) : c1 / s.AMU / s.RQ;
+            if (K >= s.itermax) {
+                s.ier = 3000;
+                s.kout = K + 1;
+                s.done = 1;
                 return;
             }
         }
     }
     if (stop) {
-        sc->kout = K;
-        sc->done = 1;
+        s.kout = K;
+        s.done = 1;
     }
+}
+
+__global__ void __launch_bounds__(FIN_BS)
+k_fin_beta(Scal *sc, const double *__restrict__ part, int G) {
+    if (sc->done) return;
+    Scal n = *sc;
+    double r[2];
+    fin_sums<2>(part, G, r);
+    if (threadIdx.x != 0) return;
+    beta_step(n, r[0], r[1]);
+    *sc = n;
 }
 
 // Mixed precision, outer step: ERR64 = sqrt(RN/BN) of the true preconditioned

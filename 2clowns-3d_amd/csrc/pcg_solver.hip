@@ -6,8 +6,8 @@
 // stays resident in HBM between solves (the SMAC pass loop of
 // src2LOWNS/1sub-momentum.F90:42-60 changes only the right-hand side), and a
 // solve runs entirely on one HIP stream.  Convergence is decided on the
-// device (k_fin_beta); the host only polls a pinned copy of the scalars every
-// few iterations, so iterations run back to back without host round trips.
+// device (beta_step); the host only polls a word that the kernels post, so
+// iterations run back to back without host round trips.
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
@@ -32,6 +32,7 @@
 #include "clowns_pcg.h"
 #include "pcg_kernels.hpp"
 #include "run_kernels.hpp"
+#include "small_kernels.hpp"
 #include "assembly_kernels.hpp"
 #include "classify_kernels.hpp"
 #include "vof_kernels.hpp"
@@ -86,6 +87,8 @@ template <typename T> struct DevBuf {
 // Vectors of one precision for one Bi-CGSTAB run.
 template <typename T> struct VecSet {
     DevBuf<T> r, rh, p0, q, e, v, y, t, x;
+    DevBuf<T> p1;  // the second P of the small kernels, padded like the others
+    int padP1 = -1;
     int padN = -1;  // the row count whose ghost rows [N, N+64) were last zeroed
     int ensure(size_t n) {
         DevBuf<T> *all[] = {&r, &rh, &p0, &q, &e, &v, &y, &t, &x};
@@ -98,7 +101,8 @@ template <typename T> struct VecSet {
     void release() {
         DevBuf<T> *all[] = {&r, &rh, &p0, &q, &e, &v, &y, &t, &x};
         for (auto *b : all) b->release();
-        padN = -1;
+        p1.release();
+        padN = padP1 = -1;
     }
 };
 
@@ -261,9 +265,23 @@ struct Knobs {
     // CLOWNS_RUNS = 0 off, 1 on wherever there are patterns; -1 (default): from
     // RUN_MIN_ROWS rows, unless a switch names a form of the kernels they replace.
     int runs = -1;
+    // The small kernels (small_kernels.hpp).  CLOWNS_SMALL = 0 never, 1 all of
+    // them and 2 with the column kernels' PM as far as they go (1,048,576 rows);
+    // -1 (default): by the limits below, unless a switch names a form of the
+    // kernels they replace.
+    int small = -1;
     // CLOWNS_VERBOSE = 1: report per-operator tuning decisions on stderr.
     bool verbose = false;
 };
+// Rows up to which an iteration is five launches (small_kernels.hpp), and up to
+// which it is nine, with the column kernels' PM.  Solves to 1e-8 in ms, single
+// kernels / nine launches / five: FP64 3.6/2.6/2.3 at 78 thousand rows,
+// 3.8/3.1/3.1 at 136, 4.4/3.9/4.9 at 217, 6.2/5.7/7.6 at 306, 5.1/5.1/6.9 at 386,
+// 6.5/7.2/10.2 at 461; mixed 4.4/3.0/2.6 at 136, 5.0/3.9/3.7 at 217, 5.6/4.8/5.1 at
+// 386, 8.1/7.5 at 574, 7.5/7.3 at 720, 8.3/9.3 at 864.  Past them the work that
+// stands in for the launches costs more than they do.
+template <typename T> constexpr int SMALL_ROWS = sizeof(T) == 8 ? 120000 : 300000;
+template <typename T> constexpr int FUSED_ROWS = sizeof(T) == 8 ? 360000 : 700000;
 
 struct clowns_solver {
     Knobs kn;
@@ -360,9 +378,16 @@ struct clowns_solver {
     DevBuf<double> vof_term;   // VOF update: quvwf_modify correction per cell
     DevBuf<int> vof_cnt;       // VOF update: flags and counters (VC_*)
     DevBuf<Scal> sc;       // [0] inner/FP64 run, [1] outer (mixed)
-    Scal *h_sc = nullptr;  // pinned mirror: [0] inner/FP64 run, [1] outer, [2], [3] poll slots
+    Scal *h_sc = nullptr;  // pinned mirror: [0] inner/FP64 run, [1] outer, [2] the polled word (run_word)
+    unsigned long long *run_word() const { return reinterpret_cast<unsigned long long *>(h_sc + 2); }
+    // The small kernels' records of the forward operator (FP64, FP32) and of
+    // the transposed one, and their dot partials.
+    struct Small {
+        DevBuf<unsigned char> mem;
+        bool ok = false;
+    } small64, small32, smallt;
+    DevBuf<double> small_part;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
-    hipEvent_t evp[2] = {nullptr, nullptr};  // ends of the two queued iteration batches
 
     // mixed: smallest relative tolerance of an inner solve.  Short inner
     // solves restart Bi-CGSTAB from the true residual more often, which on
@@ -372,7 +397,7 @@ struct clowns_solver {
     // per time step at 26M rows; 2e-2 .. 1e-1 and 3e-4 were slower.
     double tau_min = 1e-2;
     bool cls_force_host = false;  // test hook: always take the exact host path
-    int poll = 8;          // iterations between host polls of `done`
+    int poll = 3;          // iterations queued ahead of the last one seen done
     int will_max_rounds = 4096;  // PCGPME_WILL output pass: device rounds before the host pass
     int fuse64 = -1, fuse32 = -1;      // pairwise PM fusion chosen by tune_fuse ...
     int fuse64_N = 0, fuse32_N = 0;    // ... for operators of about this many rows (tuned_size)
@@ -410,8 +435,6 @@ int ensure_events(clowns_solver *h) {
         HIPCHK(hipEventCreate(&h->ev0));
         HIPCHK(hipEventCreate(&h->ev1));
         HIPCHK(hipEventCreate(&h->ev2));
-        HIPCHK(hipEventCreateWithFlags(&h->evp[0], hipEventDisableTiming));
-        HIPCHK(hipEventCreateWithFlags(&h->evp[1], hipEventDisableTiming));
     }
     return CLOWNS_OK;
 }
@@ -425,8 +448,8 @@ size_t part_len(int N) { return (size_t)2 * geo_of(N, 1).G; }
 int ensure_common(clowns_solver *h, int N) {
     int rc;
     if ((rc = h->part.ensure(part_len(N)))) return rc;
-    if ((rc = h->sc.ensure(2))) return rc;
-    if (!h->h_sc) HIPCHK(hipHostMalloc((void **)&h->h_sc, 4 * sizeof(Scal), hipHostMallocDefault));
+    if ((rc = h->sc.ensure(3))) return rc;
+    if (!h->h_sc) HIPCHK(hipHostMalloc((void **)&h->h_sc, 3 * sizeof(Scal), hipHostMallocDefault));
     return ensure_events(h);
 }
 
@@ -461,6 +484,8 @@ template <typename T> struct Op {
     bool pc2 = false;               // FP64 PM stages as k_pm_p2 (with pid; tune_stream)
     RunOp<T> run = {};              // row runs; spmv null: none
     RunGrid run_grid = {0, 0, 0};
+    SmallOp<T> small = {};          // records of the small kernels; p01 null: none
+    int small_G = 0;                // 4 small_G wavefronts leave dot partials
     KProf *prof = nullptr;          // armed kernel profile, or null
 };
 
@@ -930,7 +955,7 @@ template <typename T> void tune_stream(clowns_solver *h, Op<T> &A, VecSet<T> &V)
         Op<T> B = A;
         set_forms(B, form);
         for (int it = 0; it < 2; ++it) {
-            k_pupd_vec<T><<<Gv, BS, 0, s>>>(sc, A.N, V.p0.p, V.r.p, V.q.p);
+            k_pupd_vec<T><<<Gv, BS, 0, s>>>(sc, A.N, V.p0.p, V.r.p, V.q.p, nullptr);
             spmv<T>(s, sc, B, 0, V.p0.p, nullptr, V.y.p);
             apply_pm<T>(s, sc, B, V.y.p, V.q.p, V.y.p, V.t.p, 1, V.rh.p, part);
             k_eupd_vec<T><<<Gv, BS, 0, s>>>(sc, A.N, V.r.p, V.q.p, V.e.p);
@@ -995,62 +1020,71 @@ template <typename T> void known_stream(const clowns_solver *h, Op<T> &A) {
     if (!A.run.spmv && stored_forms(h, A, &f)) set_forms(A, f);
 }
 
-// How many iterations to enqueue next.  The device decides convergence
-// (k_fin_beta sets `done`, after which every kernel returns at once), so the
-// host only chooses how far ahead of the last status it has seen to run:
-// too short and the GPU idles while the host waits, too long and the
-// iterations queued past convergence each cost a dozen empty launches.  From
-// the residual at the last two statuses the host predicts the iteration at
-// which sqrt(RN/BN) reaches EPS (Bi-CGSTAB converges about geometrically)
-// and queues up to it; without a prediction the batch doubles, up to 32.
-struct PollPlan {
-    int n = 8;                          // last batch length
-    int k0 = 0, k1 = 0;                 // iterations of the last two statuses seen
-    double e0 = 0.0, e1 = 0.0;          // their ERR
-    // status after iteration k: ERR err, target eps
-    void seen(int k, double err) {
-        if (k1 > 0 && k - k1 < 4) return;  // too close to the last one for a slope
-        k0 = k1;
-        e0 = e1;
-        k1 = k;
-        e1 = err;
-    }
-    // length of the batch that starts at iteration `next` (statuses seen up
-    // to k1; iterations k1+1 .. next-1 already queued)
-    int next_len(int next, double eps) {
-        int len = std::min(32, 2 * n);
-        if (k0 > 0 && e0 > 0.0 && e1 > 0.0 && e1 < e0 && eps > 0.0) {
-            const double rate = std::log(e0 / e1) / (double)(k1 - k0);
-            const double left = e1 > eps ? std::log(e1 / eps) / rate : 0.0;
-            const double stop = (double)k1 + left;  // predicted last iteration
-            const double want = std::ceil(stop - (double)next + 1.0);
-            len = !(want < 32.0) ? 32 : (want <= 2.0 ? 2 : (int)want);  // NaN: 32
-        }
-        n = len;
-        return len;
-    }
-};
-
 // The PCGPME iteration (pcgpme_para.F90:148-247) on already initialised
-// vectors: V.p0 = V.r = V.rh = r0, V.x = x0, scalars BN/C1 set by k_fin_init.
-// Batches of iterations are queued one ahead of the status the host reads
-// (two pinned status slots), so the stream never drains while the host
-// looks.  Returns after the device has set `done`; the final scalars are in
-// h->h_sc[sc_index].  eps: the run's stopping value (for the batch plan only).
+// vectors: V.p0 = V.r = V.rh = r0, V.x = x0, scalars BN/C1 set by k_fin_init,
+// h->run_word cleared before that.  Returns with the stream drained after the
+// device has set `done`; the final scalars are in h->h_sc[sc_index].
 template <typename T>
-int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int itermax, int sc_index,
-                 double eps) {
+int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int itermax, int sc_index) {
     hipStream_t s = h->stream;
     double *part = h->part.p;
     const int Gv = geo_of(A.N, VecOf<T>::R).G;
     KProf *pf = A.prof;
     if (pf) pf->run = (int)pf->kout.size();
+    unsigned long long *host = h->run_word();
+    const bool small = A.small_G > 0;
+    // the small kernels' scalars and P alternate: an iteration's first kernel
+    // reads the ones before and writes its own
+    auto scal = [&](int K) { return small && K % 2 == 0 ? h->sc.p + 2 : sc; };
+    auto iteration_small = [&](int K) {
+        if (pf) pf->K = K;
+        Scal *S = scal(K);
+        const int G = A.small_G, G1 = geo_of(A.N, 1).G;
+        double *wp = h->small_part.p, *wo = wp + 8 * (size_t)G;
+        const bool rec = A.small.p01 != nullptr;
+        T *P[2] = {V.p0.p, V.p1.p};
+        T *p = P[(K + 1) % 2];
+        const T *none = nullptr;
+        unsigned long long *quiet = nullptr;
+        auto pm = [&](const T *w, T *out, auto dot) {
+            constexpr int DOT = decltype(dot)::value;
+            if (!rec) {
+                apply_pm<T>(s, S, A, V.y.p, out, V.y.p, V.t.p, DOT, w, wp);
+                return;
+            }
+            KScope ks(pf, kcls<T>(KC_PMDOT));
+            klaunch(k_small_pm<T, DOT>, 4 * G, sizeof(T) == 8 ? 128 : 256, s, S, A.N, A.small, V.y.p, out, w, wp);
+        };
+        {
+            KScope ks(pf, kcls<T>(KC_SPMV));
+            if (K == 1)
+                klaunch(k_small_spmv<T, 0, 4>, G1, BS, s, S, S, quiet, A.N, wp, 0, A.small, p, none, none, p, V.y.p);
+            else
+                klaunch(k_small_spmv<T, 1, 4>, G1, BS, s, scal(K - 1), S, host, A.N, wo, G, A.small, V.r.p, P[K % 2],
+                        V.q.p, p, V.y.p);
+        }
+        pm(V.rh.p, V.q.p, std::integral_constant<int, 1>());
+        {
+            KScope ks(pf, kcls<T>(KC_SPMV));
+            auto go = [&](auto kern) {
+                klaunch(kern, G1, BS, s, S, S, quiet, A.N, wp, G, A.small, V.r.p, none, V.q.p, V.e.p, V.y.p);
+            };
+            rec ? go(k_small_spmv<T, 2, 4>) : go(k_small_spmv<T, 2, 1>);
+        }
+        pm(V.e.p, V.v.p, std::integral_constant<int, 2>());
+        KScope ks(pf, kcls<T>(KC_UPDATE));
+        auto go = [&](auto kern) {
+            klaunch(kern, G, BS, s, S, A.N, wp, G, V.x.p, p, V.e.p, V.v.p, V.r.p, V.rh.p, wo);
+        };
+        rec ? go(k_small_update<T, 4>) : go(k_small_update<T, 1>);
+    };
     auto iteration = [&](int K) {
+        if (small) return iteration_small(K);
         if (pf) pf->K = K;
         // Q = PM*A*P (:149-151), after P = R + BETA*(P - AMU*Q) (:244) for K > 1.
         if (K > 1) {
             KScope ks(pf, kcls<T>(KC_PUPD));
-            klaunch(k_pupd_vec<T>, Gv, BS, s, sc, A.N, V.p0.p, V.r.p, V.q.p);
+            klaunch(k_pupd_vec<T>, Gv, BS, s, sc, A.N, V.p0.p, V.r.p, V.q.p, host);
         }
         spmv<T>(s, sc, A, 0, V.p0.p, nullptr, V.y.p);
         const int Gq = apply_pm<T>(s, sc, A, V.y.p, V.q.p, V.y.p, V.t.p, 1, V.rh.p, part);
@@ -1074,44 +1108,44 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
             klaunch(k_update_vec<T>, Gv, BS, s, sc, A.N, V.x.p, V.p0.p, V.e.p, V.v.p, V.r.p, V.rh.p, part);
         }
         KScope ks(pf, kcls<T>(KC_FIN));
-        klaunch(k_fin_beta, 1, FIN_BS, s, sc, part, Gv, K);
+        klaunch(k_fin_beta, 1, FIN_BS, s, sc, part, Gv);
     };
-    Scal *slot[2] = {h->h_sc + 2, h->h_sc + 3};
-    PollPlan plan;
-    plan.n = std::max(1, h->poll) / 2;
-    int K = 1;
-    auto enqueue = [&](int len, int si) -> int {
-        const int kend = std::min(itermax, K + len - 1);
-        for (; K <= kend; ++K) iteration(K);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(slot[si], sc, sizeof(Scal), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipEventRecord(h->evp[si], s));
-        return CLOWNS_OK;
-    };
-    int rc, cur = 0;
-    if ((rc = enqueue(plan.next_len(K, eps), cur))) return rc;
-    for (;;) {
-        const bool ahead = K <= itermax;
-        if (ahead && (rc = enqueue(plan.next_len(K, eps), cur ^ 1))) return rc;
-        HIPCHK(hipEventSynchronize(h->evp[cur]));
-        const Scal hs = *slot[cur];
-        if (hs.done) {
-            // a batch queued behind the converged one only returns at once
-            h->h_sc[sc_index] = hs;
-            if (ahead) {
-                HIPCHK(hipEventSynchronize(h->evp[cur ^ 1]));
-                h->h_sc[sc_index] = *slot[cur ^ 1];
-            }
-            break;
+    // The device decides convergence (after it every kernel returns at once)
+    // and posts the iterations done and the decision to a word of host memory,
+    // in the next iteration's first kernel (at the end of k_fin_beta, whose own
+    // end then waits for the host's memory, it cost 2 us an iteration).
+    // The host queues h->poll iterations ahead of the last one it saw there:
+    // enough that the GPU never waits for it, and few to run out at the end.
+    int K = 1, seen = 0;
+    const int last = itermax + 1;  // whose first kernel posts the last iteration's word
+    bool done = itermax <= 0;  // PCGPME_WILL may ask for none
+    int spins = 0;
+    while (!done) {
+        const int k0 = K;
+        while (K <= last && K - 1 - seen < h->poll) iteration(K++);
+        if (K != k0) HIPCHK(hipGetLastError());
+        const unsigned long long w = __atomic_load_n(host, __ATOMIC_RELAXED);
+        const int k = (int)(w >> 33);
+        done = (w >> 32 & 1) != 0;
+        if (done || k != seen) {
+            seen = k;
+            spins = 0;
+            continue;
         }
-        if (!ahead) {
-            // unreachable: the device sets done at itermax
-            h->h_sc[sc_index] = hs;
-            break;
+        if (++spins < 20000) {
+            __builtin_ia32_pause();
+            continue;
         }
-        plan.seen(hs.K, hs.ERR);
-        cur ^= 1;
+        spins = 0;
+        const hipError_t q = hipStreamQuery(s);
+        if (q == hipErrorNotReady) continue;
+        HIPCHK(q);
+        // the queue ran dry: the word was posted before that
+        const unsigned long long w2 = __atomic_load_n(host, __ATOMIC_RELAXED);
+        if (w2 == w) return CLOWNS_EHIP;  // unreachable: the device sets done at itermax
     }
+    HIPCHK(hipMemcpyAsync(h->h_sc + sc_index, scal(seen + 1), sizeof(Scal), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
     if (pf) {
         pf->kout.push_back(h->h_sc[sc_index].kout);
         pf->run = -1;
@@ -1439,6 +1473,42 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     return build_forms(h);
 }
 
+// Whether the small kernels run the resident operator in this precision: with
+// the column kernels' PM, or all of them.
+template <typename T> bool fused_size(const clowns_solver *h) {
+    if (h->NL != 6 || h->kn.small == 0 || geo_of(h->N, 2).G > SMALL_MAX_G || !h->kn.v4_32) return false;
+    return h->kn.small > 0 || h->N <= FUSED_ROWS<T>;
+}
+template <typename T> bool small_size(const clowns_solver *h) {
+    return fused_size<T>(h) && (h->kn.small < 0 ? h->N <= SMALL_ROWS<T> : h->kn.small == 1);
+}
+// The small kernels' records of an operator's columns.
+template <typename T, typename C>
+int build_small(clowns_solver *h, clowns_solver::Small &m, const C *AL, const int *LL) {
+    const size_t n = (size_t)h->N + 1;
+    int rc;
+    m.ok = false;
+    if ((rc = m.mem.ensure(n * (2 * sizeof(SmallPair<T>) + sizeof(SmallLast<T>))))) return rc;
+    SmallPair<T> *p01 = reinterpret_cast<SmallPair<T> *>(m.mem.p);
+    k_small_build<T, C><<<cdiv((long)n, BS), BS, 0, h->stream>>>(h->N, h->lda, AL, LL, p01, p01 + n,
+                                                                 reinterpret_cast<SmallLast<T> *>(p01 + 2 * n));
+    HIPCHK(hipGetLastError());
+    m.ok = true;
+    return CLOWNS_OK;
+}
+template <typename T> void use_small(const clowns_solver *h, const clowns_solver::Small &m, Op<T> &A) {
+    if (!m.ok) {
+        if (fused_size<T>(h) && !h->run_ok) {
+            A.small = {A.AL, A.D, A.LL, A.lda, nullptr, nullptr, nullptr};
+            A.small_G = geo_of(A.N, sizeof(T) == 8 ? 2 : 4).G;
+        }
+        return;
+    }
+    const size_t n = (size_t)A.N + 1;
+    const SmallPair<T> *p01 = reinterpret_cast<const SmallPair<T> *>(m.mem.p);
+    A.small = {A.AL, A.D, A.LL, A.lda, p01, p01 + n, reinterpret_cast<const SmallLast<T> *>(p01 + 2 * n)};
+    A.small_G = geo_of(A.N, sizeof(T) == 8 ? 2 : 4).G;
+}
 int ensure_f32(clowns_solver *h) {
     if (h->have32) return CLOWNS_OK;
     int rc;
@@ -1453,6 +1523,11 @@ int ensure_f32(clowns_solver *h) {
     h->have_h = h->kn.pm_half;
     h->have_rows = h->have_rows8 = false;
     if ((rc = build_runs32(h))) return rc;
+    h->small32.ok = false;
+    if (small_size<float>(h) && !h->run_ok &&
+        (rc = h->have_h ? build_small<float, _Float16>(h, h->small32, h->ALh.p, h->LL.p)
+                        : build_small<float, float>(h, h->small32, h->AL32.p, h->LL.p)))
+        return rc;
     if (h->kn.rows32 && h->NL == 6 && h->ll16_ok && !h->run_ok) {
         const size_t n6 = (size_t)6 * h->N;
         if ((rc = h->ALr32.ensure(n6)) || (rc = h->Lr16.ensure(n6)) || (rc = h->nonunit.ensure(1))) return rc;
@@ -1691,6 +1766,13 @@ int build_runs(clowns_solver *h) {
 // patterns, then the row runs, or the index codes of the column kernels.
 int build_forms(clowns_solver *h) {
     int rc;
+    h->small64.ok = false;
+    if (small_size<double>(h)) {
+        if ((rc = build_small<double, double>(h, h->small64, h->AL.p, h->LL.p))) return rc;
+        h->pat_ok = h->run_ok = h->ll16_ok = h->ll8_ok = false;
+        h->pat_rows = 0;
+        return CLOWNS_OK;
+    }
     if ((rc = build_patterns(h)) || (rc = build_runs(h))) return rc;
     h->ll16_ok = h->ll8_ok = false;
     h->ll16_wide = h->ll8_wide = 0;
@@ -1782,6 +1864,7 @@ Op<double> op64(const clowns_solver *h) {
         A.pid = h->pid.p;
         A.ptab = h->ptab.p;
     }
+    use_small(h, h->small64, A);
     use_runs(h, A);
     return A;
 }
@@ -1815,6 +1898,7 @@ Op<float> op32(const clowns_solver *h) {
             A.base8 = nullptr;
         }
     }
+    if (h->have32) use_small(h, h->small32, A);
     use_runs(h, A);
     return A;
 }
@@ -1842,6 +1926,23 @@ template <typename T> int ensure_vecs(clowns_solver *h, VecSet<T> &V, int N) {
     return CLOWNS_OK;
 }
 
+// The small kernels' second P and dot partials; without room for them the
+// single kernels run.
+template <typename T> int ensure_small(clowns_solver *h, VecSet<T> &V, Op<T> &A) {
+    if (!A.small_G) return CLOWNS_OK;
+    if (V.p1.ensure((size_t)A.N + VEC_PAD) || h->small_part.ensure(16 * (size_t)geo_of(A.N, 2).G)) {
+        (void)hipGetLastError();
+        A.small = {};
+        A.small_G = 0;
+        return CLOWNS_OK;
+    }
+    if (V.padP1 != A.N) {
+        fill<T>(h->stream, V.p1.p + A.N, VEC_PAD, T(0));
+        V.padP1 = A.N;
+    }
+    return CLOWNS_OK;
+}
+
 // The scaled right-hand side of a run (the mixed solve gathers it in its
 // first PM application): N + 64 entries, ghost rows zero.
 int ensure_bs(clowns_solver *h, int N) {
@@ -1865,7 +1966,8 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
     VecSet<double> &V = h->v64;
     if ((rc = ensure_vecs(h, V, A_in.N)) || (rc = ensure_bs(h, A_in.N))) return rc;
     Op<double> A = A_in;
-    if (!A.run.spmv) {
+    if ((rc = ensure_small(h, V, A))) return rc;
+    if (!A.run.spmv && !A.small.p01) {
         A.fuse = tune_fuse(h, A, V);
         tune_stream(h, A, V);
     }
@@ -1888,10 +1990,11 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
         wk3 = V.q.p;
     }
     k_init<double><<<G1, BS, 0, s>>>(sc, N, V.p0.p, wk3, V.r.p, V.rh.p, part);
-    k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1);
+    *h->run_word() = 0;
+    k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1, h->run_word());
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(h->ev2, s));
-    if ((rc = run_bicgstab<double>(h, A, V, sc, itermax, 0, eps))) return rc;
+    if ((rc = run_bicgstab<double>(h, A, V, sc, itermax, 0))) return rc;
     HIPCHK(hipMemcpyAsync(d_x, V.x.p, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, s));
     HIPCHK(hipEventRecord(h->ev1, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -1925,12 +2028,12 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
         return rc;
     Op<double> A = A_in;
     Op<float> A32 = A32_in;
-    if (!A.run.spmv) {
-        A.fuse = tune_fuse(h, A, V);
-        A32.fuse = tune_fuse(h, A32, F);
-        tune_stream(h, A, V);
-        tune_stream(h, A32, F);
-    }
+    if ((rc = ensure_small(h, F, A32))) return rc;
+    const bool t64 = !A.run.spmv && !A.small.p01, t32 = !A.run.spmv && !A32.small.p01;
+    if (t64) A.fuse = tune_fuse(h, A, V);
+    if (t32) A32.fuse = tune_fuse(h, A32, F);
+    if (t64) tune_stream(h, A, V);
+    if (t32) tune_stream(h, A32, F);
     if (h->prof.on) A.prof = A32.prof = &h->prof;
     const int N = A.N;
     const int G1 = geo_of(N, 1).G;
@@ -1985,8 +2088,9 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
             k_rhs32<<<cdiv(N, BS), BS, 0, s>>>(N, outer, V.r.p, F.p0.p);
             fill<float>(s, F.x.p, (size_t)N, 0.f);
             k_init<float><<<G1, BS, 0, s>>>(sc, N, F.p0.p, nullptr, F.r.p, F.rh.p, part);
-            k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1);
-            if ((rc = run_bicgstab<float>(h, A32, F, sc, std::max(1, itermax - total_inner), 0, tau)))
+            *h->run_word() = 0;
+            k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1, h->run_word());
+            if ((rc = run_bicgstab<float>(h, A32, F, sc, std::max(1, itermax - total_inner), 0)))
                 return rc;
             total_inner += std::max(0, std::min(h->h_sc[0].kout, itermax));
             ++refinements;
@@ -2081,10 +2185,14 @@ extern "C" int clowns_solver_create(clowns_solver **out, int device, void *strea
         flag("CLOWNS_VERBOSE", k.verbose);
         flag("CLOWNS_PATTERNS", k.patterns);
         tri("CLOWNS_RUNS", k.runs);
-        if (k.runs < 0)
+        if (const char *e = getenv("CLOWNS_SMALL")) k.small = std::min(2, std::max(-1, atoi(e)));
+        if (k.runs < 0 || k.small < 0)
             for (const char *name : {"CLOWNS_FUSE_PM", "CLOWNS_STREAM", "CLOWNS_LL8", "CLOWNS_PM_PAT", "CLOWNS_LL16",
                                      "CLOWNS_V4_32", "CLOWNS_SPMV_ROWS", "CLOWNS_SPMV32_P2"})
-                if (getenv(name)) k.runs = 0;
+                if (getenv(name)) {
+                    if (k.runs < 0) k.runs = 0;
+                    if (k.small < 0) k.small = 0;
+                }
         flag("CLOWNS_CLASSIFY_HOST", h->cls_force_host);
         if (const char *e = getenv("CLOWNS_POLL")) h->poll = std::max(1, atoi(e));
         if (const char *e = getenv("CLOWNS_TAU_MIN")) h->tau_min = std::max(1e-8, atof(e));
@@ -2100,6 +2208,7 @@ extern "C" int clowns_solver_destroy(clowns_solver *h) {
     (void)hipStreamSynchronize(h->stream);
     h->AL.release(); h->D.release(); h->W.release(); h->LL.release(); h->LL16.release(); h->base16.release(); h->LL8.release(); h->base8.release(); h->order.release(); h->order_first.release();
     h->AL32.release(); h->D32.release(); h->ALh.release(); h->ALr32.release(); h->Lr16.release(); h->Lr8.release(); h->nonunit.release(); h->pid.release(); h->ptab.release();
+    h->small64.mem.release(); h->small32.mem.release(); h->smallt.mem.release(); h->small_part.release();
     h->run_n.release(); h->run_raw[0].release(); h->run_raw[1].release(); h->run_raws.release(); h->run_pair[0].release(); h->run_pair[1].release(); h->run_spmv.release(); h->run_pair32[0].release(); h->run_pair32[1].release(); h->run_spmv32.release(); h->run_lj.release(); h->run_c.release(); h->run_c32.release(); h->run_cid.release(); h->run_rq.release(); h->run_wave.release(); h->run_wave32.release(); h->run_rj.release(); h->run_rc.release(); h->run_rc32.release();
     h->pat_keys.release();
     h->ALt.release(); h->Dt.release(); h->Wt.release(); h->LLt.release();
@@ -2109,7 +2218,6 @@ extern "C" int clowns_solver_destroy(clowns_solver *h) {
     h->v64.release(); h->v32.release(); h->bs.release(); h->stage_b.release(); h->stage_x.release(); h->part.release(); h->flag.release(); h->will_flags.release(); h->will_cand.release(); h->will_rev.release(); h->cls_scratch.release(); h->pc_b.release(); h->pc_x.release(); h->pc_part.release(); h->sc.release();
     if (h->h_sc) (void)hipHostFree(h->h_sc);
     if (h->ev0) { (void)hipEventDestroy(h->ev0); (void)hipEventDestroy(h->ev1); (void)hipEventDestroy(h->ev2); }
-    for (hipEvent_t e : h->evp) if (e) (void)hipEventDestroy(e);
     h->prof.release();
     if (h->own_stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -2160,15 +2268,16 @@ extern "C" int clowns_solver_solve(clowns_solver *h, const double *d_b, double *
 // (every GPU the library runs on holds its own copy until the process ends)
 // for the runs' vectors (nine FP64 and nine FP32 ones of N + 64 entries and
 // their slack, each 256-byte aligned), the scaled right-hand side, the dot
-// partials and the run scalars, for up to NOALLOC_MAX_ROWS rows: 58 MiB.
+// partials and the run scalars, for up to NOALLOC_MAX_ROWS rows: 65 MiB.
 constexpr int NOALLOC_MAX_ROWS = 1 << 19;
 constexpr size_t NA_VEC = (size_t)NOALLOC_MAX_ROWS + 704;                  // entries per vector
 constexpr size_t NA_G1 = (((size_t)NOALLOC_MAX_ROWS + BS - 1) / BS + 7) / 8 * 8;  // largest grid
-constexpr size_t NA_V64 = 0;                                                 // 9 FP64 vectors + bs
-constexpr size_t NA_V32 = NA_V64 + 10 * NA_VEC * sizeof(double);             // 9 FP32 vectors
-constexpr size_t NA_PART = NA_V32 + 9 * NA_VEC * sizeof(float);              // 2 x NA_G1 partials
-constexpr size_t NA_SC = NA_PART + 2 * NA_G1 * sizeof(double);               // 2 run scalars
-constexpr size_t NA_BYTES = NA_SC + 2 * sizeof(Scal);
+constexpr size_t NA_V64 = 0;                                                 // 10 FP64 vectors + bs
+constexpr size_t NA_V32 = NA_V64 + 11 * NA_VEC * sizeof(double);             // 10 FP32 vectors
+constexpr size_t NA_PART = NA_V32 + 10 * NA_VEC * sizeof(float);             // 2 x NA_G1 partials
+constexpr size_t NA_SPART = NA_PART + 2 * NA_G1 * sizeof(double);            // 16 a 512-row block
+constexpr size_t NA_SC = NA_SPART + 16 * (NA_G1 / 2 + 8) * sizeof(double);   // 3 run scalars
+constexpr size_t NA_BYTES = NA_SC + 3 * sizeof(Scal);
 static_assert(NA_VEC >= (size_t)NOALLOC_MAX_ROWS + VEC_PAD, "room for the zero rows");
 static_assert(NA_VEC * sizeof(float) % 256 == 0 && NA_V32 % 256 == 0 && NA_PART % 256 == 0 && NA_SC % 256 == 0,
               "vectors start 256-byte aligned");
@@ -2193,9 +2302,9 @@ int scratch_of(int dev, unsigned char **out) {
 }
 
 template <typename T> void borrow_vecs(VecSet<T> &V, unsigned char *base) {
-    DevBuf<T> *all[] = {&V.r, &V.rh, &V.p0, &V.q, &V.e, &V.v, &V.y, &V.t, &V.x};
-    for (int k = 0; k < 9; ++k) all[k]->borrow((T *)(base + (size_t)k * NA_VEC * sizeof(T)), NA_VEC);
-    V.padN = -1;  // the array keeps the last call's contents: ghost rows cleared again
+    DevBuf<T> *all[] = {&V.r, &V.rh, &V.p0, &V.q, &V.e, &V.v, &V.y, &V.t, &V.x, &V.p1};
+    for (int k = 0; k < 10; ++k) all[k]->borrow((T *)(base + (size_t)k * NA_VEC * sizeof(T)), NA_VEC);
+    V.padN = V.padP1 = -1;  // the array keeps the last call's contents: ghost rows cleared again
 }
 } // namespace
 
@@ -2214,7 +2323,7 @@ extern "C" int clowns_solver_solve_noalloc(clowns_solver *h, const double *d_b, 
         return CLOWNS_EBADARG;
     }
     // the pinned status mirror and the events come with the operator
-    if (!h->h_sc || !h->ev0 || !h->evp[0]) return CLOWNS_EBADARG;
+    if (!h->h_sc || !h->ev0) return CLOWNS_EBADARG;
     int rc = set_device(h);
     if (rc) return rc;
     unsigned char *base = nullptr;
@@ -2224,17 +2333,19 @@ extern "C" int clowns_solver_solve_noalloc(clowns_solver *h, const double *d_b, 
     // the run's work buffers point into the array for this call
     VecSet<double> v64;
     VecSet<float> v32;
-    DevBuf<double> bs, part;
+    DevBuf<double> bs, part, small_part;
     DevBuf<Scal> sc;
     borrow_vecs(v64, base + NA_V64);
-    bs.borrow((double *)(base + NA_V64 + 9 * NA_VEC * sizeof(double)), NA_VEC);
+    bs.borrow((double *)(base + NA_V64 + 10 * NA_VEC * sizeof(double)), NA_VEC);
     borrow_vecs(v32, base + NA_V32);
     part.borrow((double *)(base + NA_PART), 2 * NA_G1);
-    sc.borrow((Scal *)(base + NA_SC), 2);
+    small_part.borrow((double *)(base + NA_SPART), 16 * (NA_G1 / 2 + 8));
+    sc.borrow((Scal *)(base + NA_SC), 3);
     std::swap(h->v64, v64);
     std::swap(h->v32, v32);
     std::swap(h->bs, bs);
     std::swap(h->part, part);
+    std::swap(h->small_part, small_part);
     std::swap(h->sc, sc);
     const int bs_padN = h->bs_padN;
     const bool prof_on = h->prof.on;
@@ -2250,6 +2361,7 @@ extern "C" int clowns_solver_solve_noalloc(clowns_solver *h, const double *d_b, 
     std::swap(h->v32, v32);
     std::swap(h->bs, bs);
     std::swap(h->part, part);
+    std::swap(h->small_part, small_part);
     std::swap(h->sc, sc);
     h->bs_padN = bs_padN;
     h->prof.on = prof_on;
@@ -2725,7 +2837,13 @@ int ensure_transpose(clowns_solver *h) {
     else
         k_scale_sort<4><<<cdiv(N, BS), BS, 0, s>>>(N, lda, h->ALt.p, h->LLt.p, h->Dt.p, h->Wt.p, P1, P2);
     HIPCHK(hipGetLastError());
-    if ((rc = build_codes_t(h))) return rc;
+    h->smallt.ok = false;
+    if (h->small64.ok) {
+        h->t16_ok = h->t8_ok = false;
+        if ((rc = build_small<double, double>(h, h->smallt, h->ALt.p, h->LLt.p))) return rc;
+    } else if ((rc = build_codes_t(h))) {
+        return rc;
+    }
     h->have_t = true;
     return CLOWNS_OK;
 }
@@ -2751,6 +2869,7 @@ extern "C" int clowns_solver_solve_transpose(clowns_solver *h, const double *d_g
         At.LL8 = h->LLt8.p;
         At.base8 = h->baset8.p;
     }
+    use_small(h, h->smallt, At);
     // the transpose has the forward operator's rows: the same block order
     if (h->order_G > 0 && h->order_G == geo_of(h->N, 2).G) At.order = h->order.p;
     return solve_fp64(h, At, h->Wt.p, d_g, d_lambda, eps, maxiter,
