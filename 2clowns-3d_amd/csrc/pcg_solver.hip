@@ -374,7 +374,9 @@ struct clowns_solver {
     bool will_rev_valid = false;  // will_rev holds the readers of the resident LL0
     DevBuf<int> cls_scratch;  // classification: extents, change flag, block counts
     DevBuf<double> pc_b, pc_x, pc_part;  // pressure-correction loop: RHS, xe, DMAX partials
-    DevBuf<int> vof_state;     // VOF update: quvwf_modify state per cell
+    DevBuf<int> vof_state;     // VOF update: quvwf_modify state per surface cell
+    DevBuf<unsigned> vof_list; // the surface cells, a segment a VOF_SEG cells, and their numbers
+    DevBuf<int> vof_nlist;
     DevBuf<double> vof_term;   // VOF update: quvwf_modify correction per cell
     DevBuf<int> vof_cnt;       // VOF update: flags and counters (VC_*)
     DevBuf<Scal> sc;       // [0] inner/FP64 run, [1] outer (mixed)
@@ -2215,6 +2217,7 @@ extern "C" int clowns_solver_destroy(clowns_solver *h) {
     h->LLt16.release(); h->baset16.release(); h->LLt8.release(); h->baset8.release();
     h->AL0.release(); h->D0.release(); h->LL0.release();
     release_stager(h);
+    h->vof_state.release(); h->vof_list.release(); h->vof_nlist.release(); h->vof_term.release(); h->vof_cnt.release();
     h->v64.release(); h->v32.release(); h->bs.release(); h->stage_b.release(); h->stage_x.release(); h->part.release(); h->flag.release(); h->will_flags.release(); h->will_cand.release(); h->will_rev.release(); h->cls_scratch.release(); h->pc_b.release(); h->pc_x.release(); h->pc_part.release(); h->sc.release();
     if (h->h_sc) (void)hipHostFree(h->h_sc);
     if (h->ev0) { (void)hipEventDestroy(h->ev0); (void)hipEventDestroy(h->ev1); (void)hipEventDestroy(h->ev2); }
@@ -3239,12 +3242,12 @@ bool vof_grid_ok(const clowns_grid_dev *g) {
            g->dx && g->dt > 0.0 && g->stride >= std::max(g->nx, std::max(g->ny, g->nz)) + 2;
 }
 __global__ void k_vof_cnt_zero(int *__restrict__ cnt, int i0, int n) {
-    if ((int)threadIdx.x < n) cnt[i0 + threadIdx.x] = 0;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) cnt[i0 + k] = 0;
 }
 
-// Buffers, the device view and the flag check shared by the VOF entries;
-// on success the counters are zeroed and every flag the kernels rely on
-// for their neighbour reads has been verified on the device.
+// Buffers, the device view and the flag check shared by the VOF entries.  The
+// counters are zeroed; flags that the kernels could not rely on for their
+// neighbour reads leave VC_BAD, and then none of the update's kernels writes.
 int vof_setup(clowns_solver *h, const clowns_grid_dev *g, const double *d_Fp, double *d_qf, double *d_Fnew,
               VofDev &v, int n_plic = 0, const int32_t *d_plic_cells = nullptr) {
     if (!h || !vof_grid_ok(g) || !d_Fp || !d_qf || !d_Fnew) return CLOWNS_EBADARG;
@@ -3253,6 +3256,7 @@ int vof_setup(clowns_solver *h, const clowns_grid_dev *g, const double *d_Fp, do
     hipStream_t s = h->stream;
     const long nc = (long)(g->nx + 2) * (g->ny + 2) * (g->nz + 2);
     if ((rc = h->vof_state.ensure(nc)) || (rc = h->vof_term.ensure(nc)) || (rc = h->vof_cnt.ensure(VC_N)) ||
+        (rc = h->vof_list.ensure((size_t)cdiv(nc, VOF_SEG) * VOF_SEG)) || (rc = h->vof_nlist.ensure(cdiv(nc, VOF_SEG))) ||
         (rc = ensure_events(h)))
         return rc;
     v.nx = g->nx;
@@ -3273,12 +3277,10 @@ int vof_setup(clowns_solver *h, const clowns_grid_dev *g, const double *d_Fp, do
     v.D = h->vof_term.p;  // quvwf_modify's terms are applied before k_vof_newf writes D
     int *cnt = h->vof_cnt.p;
     k_vof_cnt_zero<<<1, 64, 0, s>>>(cnt, 0, VC_N);
-    k_vof_check<<<cdiv(nc, 256), 256, 0, s>>>(v, cnt);
+    k_vof_check<<<cdiv(nc, VOF_SEG), 64, 0, s>>>(v, cnt, h->vof_state.p, h->vof_list.p, h->vof_nlist.p);
     if (n_plic > 0) k_vof_check_plic<<<cdiv(n_plic, 256), 256, 0, s>>>(v, n_plic, d_plic_cells, cnt);
-    int bad = 0;
-    HIPCHK(hipMemcpyAsync(&bad, cnt + VC_BAD, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return bad ? CLOWNS_EBADARG : CLOWNS_OK;
+    HIPCHK(hipGetLastError());
+    return CLOWNS_OK;
 }
 
 // One cal_vof: mode 0 (PLIC face fluxes given per face, or the PLIC
@@ -3293,54 +3295,77 @@ int vof_run(clowns_solver *h, const clowns_grid_dev *g, const double *d_Fp, int3
     const long nc = v.ncell;
     int *cnt = h->vof_cnt.p;
     double dt = g->dt;
-    const int G = cdiv(nc, 256), G8 = (G + 7) & ~7, Gc8 = (cdiv((long)g->nx * g->ny, 256) + 7) & ~7;
+    const int G = cdiv(nc, 256), G8 = (G + 7) & ~7, Gc8 = (cdiv((long)g->nx * g->ny, 64) + 7) & ~7;
+    const int GL = cdiv(nc, VOF_SEG);
     clowns_vof_info out{};
     HIPCHK(hipEventRecord(h->ev0, s));
     // cal_quvwf with the surface stage
     if (mode == 1)
-        k_vof_flux<1><<<G8, 256, 0, s>>>(v, dt, nullptr, nullptr);
+        k_vof_flux<1><<<G8, 256, 0, s>>>(v, dt, nullptr, nullptr, cnt);
     else
-        k_vof_flux<0><<<G8, 256, 0, s>>>(v, dt, d_qs, d_qs_mask);
-    if (n_plic > 0) k_vof_plic<<<cdiv(n_plic, 256), 256, 0, s>>>(v, dt, n_plic, d_plic_cells, d_plic_vol);
+        k_vof_flux<0><<<G8, 256, 0, s>>>(v, dt, d_qs, d_qs_mask, cnt);
+    if (n_plic > 0) k_vof_plic<<<cdiv(n_plic, 256), 256, 0, s>>>(v, dt, n_plic, d_plic_cells, d_plic_vol, cnt);
     // quvwf_modify: rounds until every surface cell is decided (each round
-    // decides at least the first pending cell of the serial order)
-    k_vof_state_init<<<G, 256, 0, s>>>(nc, h->vof_state.p);
-    for (int round = 1;; ++round) {
-        k_vof_cnt_zero<<<1, 64, 0, s>>>(cnt, VC_PENDING, 1);
-        k_vof_mod_eval<<<G, 256, 0, s>>>(v, dt, round, h->vof_state.p, h->vof_term.p, cnt);
-        int pending = 0;
-        HIPCHK(hipMemcpyAsync(&pending, cnt + VC_PENDING, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        out.rounds = round;
-        if (pending == 0) break;
-        if (round >= (1 << 29)) return CLOWNS_EHIP;  // unreachable: every round decides a cell
-    }
-    k_vof_mod_apply<<<G, 256, 0, s>>>(v, h->vof_state.p, h->vof_term.p);
-    // cal_new_f, with its retry at dt/1.1 (1sub-vof.F90:256-268)
-    for (;;) {
-        k_vof_cnt_zero<<<1, 64, 0, s>>>(cnt, VC_RETRY, 2);
+    // decides at least the first pending cell of the serial order).  The first
+    // VOF_ROUNDS are queued with everything after them (a look by the host
+    // costs more than a round); what follows stands back if cells are left.
+    auto eval = [&](int round, int prev, int slot) {
+        k_vof_mod_eval<<<GL, 256, 0, s>>>(v, dt, round, h->vof_state.p, h->vof_term.p, h->vof_list.p, h->vof_nlist.p, cnt,
+                                        prev, slot);
+    };
+    auto apply = [&]() {
+        k_vof_mod_apply<<<GL, 256, 0, s>>>(v, h->vof_state.p, h->vof_term.p, h->vof_list.p, h->vof_nlist.p, cnt);
+    };
+    // cal_new_f's pass, then simple_slide(0) (SLIDE0 builds) unless it asks for
+    // another
+    auto rest = [&]() {
         k_vof_newf<<<G8, 256, 0, s>>>(v, dt, cnt);
-        int fl[2] = {0, 0};
-        HIPCHK(hipMemcpyAsync(fl, cnt + VC_RETRY, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        if (fl[1]) return CLOWNS_EVOF;  // the reference STOPs (F > F_lim on a surface cell)
-        if (!fl[0]) break;
+        k_vof_slide<<<Gc8, 64, 0, s>>>(v, dt, cnt);
+    };
+    int c8[VC_N];
+    auto look = [&]() -> int {
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(c8, cnt, sizeof(c8), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipEventRecord(h->ev1, s));
+        HIPCHK(hipEventSynchronize(h->ev1));
+        return CLOWNS_OK;
+    };
+    static_assert(VOF_ROUNDS >= 2 && VC_ROUND + VOF_ROUNDS - 1 <= VC_N, "a counter a round, the last one VC_PENDING");
+    for (int r = 1; r <= VOF_ROUNDS; ++r)
+        eval(r, r > 1 ? VC_ROUND + r - 2 : -1, r < VOF_ROUNDS ? VC_ROUND + r - 1 : VC_PENDING);
+    apply();
+    rest();
+    if ((rc = look())) return rc;
+    if (c8[VC_BAD]) return CLOWNS_EBADARG;
+    out.rounds = 1;
+    while (out.rounds < VOF_ROUNDS && c8[VC_ROUND + out.rounds - 1] != 0) ++out.rounds;
+    if (c8[VC_PENDING] != 0) {
+        do {
+            if (out.rounds >= (1 << 29)) return CLOWNS_EHIP;  // unreachable: every round decides a cell
+            k_vof_cnt_zero<<<1, 64, 0, s>>>(cnt, VC_PENDING, 1);
+            eval(++out.rounds, -1, VC_PENDING);
+            if ((rc = look())) return rc;
+        } while (c8[VC_PENDING] != 0);
+        apply();
+        rest();
+        if ((rc = look())) return rc;
+    }
+    // cal_new_f's retry at dt/1.1 (1sub-vof.F90:256-268)
+    for (;;) {
+        if (c8[VC_STOP]) return CLOWNS_EVOF;  // the reference STOPs (F > F_lim on a surface cell)
+        if (!c8[VC_RETRY]) break;
         dt = dt / 1.1;
         ++out.retries;
         if (dt < VOF_DTLIM) return CLOWNS_EVOF;
+        k_vof_cnt_zero<<<1, 64, 0, s>>>(cnt, VC_RETRY, 2);
+        rest();
+        if ((rc = look())) return rc;
     }
-    // simple_slide(0) (SLIDE0 builds)
-    k_vof_slide<<<Gc8, 256, 0, s>>>(v, dt, cnt);
-    HIPCHK(hipGetLastError());
-    int c8[VC_N];
-    HIPCHK(hipMemcpyAsync(c8, cnt, sizeof(c8), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipEventRecord(h->ev1, s));
-    HIPCHK(hipEventSynchronize(h->ev1));
     if (c8[VC_SOLID]) return CLOWNS_ENONFINITE;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, h->ev0, h->ev1);
     out.modified = c8[VC_MODIFIED];
-    out.slid = c8[VC_SLID];
+    for (int k = 0; k < VC_SLOTS; ++k) out.slid += c8[VC_SLID + VC_LINE * k];
     out.dt = dt;
     out.ms = ms;
     if (info) *info = out;
@@ -3371,12 +3396,16 @@ extern "C" int clowns_solver_vof_time_kernel(clowns_solver *h, const clowns_grid
     int rc = vof_setup(h, g, d_Fp, d_qf, d_Fnew, v);
     if (rc) return rc;
     hipStream_t s = h->stream;
-    const int G8 = (cdiv(v.ncell, 256) + 7) & ~7, Gc8 = (cdiv((long)v.nx * v.ny, 256) + 7) & ~7;
+    int bad = 0;
+    HIPCHK(hipMemcpyAsync(&bad, h->vof_cnt.p + VC_BAD, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (bad) return CLOWNS_EBADARG;
+    const int G8 = (cdiv(v.ncell, 256) + 7) & ~7, Gc8 = (cdiv((long)v.nx * v.ny, 64) + 7) & ~7;
     auto launch = [&]() {
         switch (kernel) {
-        case 0: k_vof_flux<1><<<G8, 256, 0, s>>>(v, g->dt, nullptr, nullptr); break;
+        case 0: k_vof_flux<1><<<G8, 256, 0, s>>>(v, g->dt, nullptr, nullptr, h->vof_cnt.p); break;
         case 1: k_vof_newf<<<G8, 256, 0, s>>>(v, g->dt, h->vof_cnt.p); break;
-        case 2: k_vof_slide<<<Gc8, 256, 0, s>>>(v, g->dt, h->vof_cnt.p); break;
+        case 2: k_vof_slide<<<Gc8, 64, 0, s>>>(v, g->dt, h->vof_cnt.p); break;
         default: k_copy<double><<<cdiv(v.ncell, BS), BS, 0, s>>>((int)v.ncell, g->F, d_Fnew); break;
         }
     };

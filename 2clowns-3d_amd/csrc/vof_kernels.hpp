@@ -58,74 +58,126 @@ __device__ __forceinline__ int vof_block() {
 
 // counters: [0] retry (cal_new_f's icon = 30), [1] stop (F > F_lim on a
 // surface cell), [2] correction aimed at a solid cell, [3] pending cells of
-// a modify round, [4] corrected cells, [5] slid cells, [6] invalid flags
-enum { VC_RETRY = 0, VC_STOP = 1, VC_SOLID = 2, VC_PENDING = 3, VC_MODIFIED = 4, VC_SLID = 5, VC_BAD = 6,
-       VC_N = 8 };
+// the last modify round, [4] corrected cells, [6] invalid flags, [8..] pending
+// cells of the first rounds, [16..] slid cells, in VC_SLOTS counters of a cache
+// line each: atomics on one address take their turns, some 50 ns each, which
+// cost k_vof_slide 8 us (a wavefront's count each)
+enum { VC_RETRY = 0, VC_STOP = 1, VC_SOLID = 2, VC_PENDING = 3, VC_MODIFIED = 4, VC_BAD = 6, VC_ROUND = 8,
+       VC_SLID = 16, VC_SLOTS = 64, VC_LINE = 16, VC_N = VC_SLID + VC_SLOTS * VC_LINE };
+constexpr int VOF_ROUNDS = 2;  // modify rounds queued before the host looks
 
-__device__ inline void vof_pos(const VofDev &v, long c, int p[3]) {
-    const int X = v.nx + 2, Y = v.ny + 2;
-    p[0] = (int)(c % X);
-    p[1] = (int)((c / X) % Y);
-    p[2] = (int)(c / ((long)X * Y));
+// The kernels of an update are queued together; each goes ahead only if what
+// came before it did not end the update: valid flags, then (from the
+// corrections on) no pending cell, then (simple_slide) no retry and no stop.
+__device__ __forceinline__ bool vof_valid(const int *cnt) { return cnt[VC_BAD] == 0; }
+__device__ __forceinline__ bool vof_settled(const int *cnt) { return (cnt[VC_BAD] | cnt[VC_PENDING]) == 0; }
+
+// Box index of a cell (they fit 32 bits: every field of a larger box would
+// outgrow the memory), in 32-bit divisions.
+__device__ __forceinline__ void vof_pos(const VofDev &v, long c, int p[3]) {
+    const unsigned X = v.nx + 2, Y = v.ny + 2, u = (unsigned)c, r = u / X;
+    p[0] = (int)(u - r * X);
+    p[2] = (int)(r / Y);
+    p[1] = (int)(r - (unsigned)p[2] * Y);
 }
 
 // df_vof(nn) = fp - dt*renzoku_fv(...) (1sub-vof.F90:271-300,
 // lib/src/math_func.F90:51-54); the low faces of c may carry a pending
-// correction of a predecessor (sub[l], applied as qf - sub).
-__device__ inline double vof_df(const VofDev &v, long c, const int p[3], double dt, const double sub[3],
-                                const bool has_sub[3]) {
+// correction of a predecessor (sub[l], applied as qf - sub).  The loads do not
+// wait for the flags: a solid neighbour's values are loaded and not used.
+struct VofCell {
+    double q[3], a[3], qh[3], ah[3], Fp, fb;
+    bool solid[3];  // the high neighbours
+};
+__device__ __forceinline__ void vof_load(const VofDev &v, long c, VofCell &w) {
     const long st[3] = {1, (long)(v.nx + 2), (long)(v.nx + 2) * (v.ny + 2)};
-    double qp[3], qm[3], ap[3], am[3];
+#pragma unroll
     for (int l = 0; l < 3; ++l) {
-        const long h = c + st[l];
+        const long h = min(c + st[l], v.ncell - 1);  // a ring cell's may lie past the box
         const size_t oc = (size_t)l * v.ncell + c, oh = (size_t)l * v.ncell + h;
-        const bool hs = v.nf[h] == -1;
-        qp[l] = hs ? 0.0 : v.qf[oh];
-        ap[l] = hs ? 0.0 : v.a[oh];
-        const double q = v.qf[oc];
-        qm[l] = has_sub[l] ? q - sub[l] : q;
-        am[l] = v.a[oc];
+        w.solid[l] = v.nf[h] == -1;
+        w.q[l] = v.qf[oc];
+        w.a[l] = v.a[oc];
+        w.qh[l] = v.qf[oh];
+        w.ah[l] = v.a[oh];
     }
-    const double r = ((qp[0] * ap[0] - qm[0] * am[0]) / v.dx[p[0]] +
-                      (qp[1] * ap[1] - qm[1] * am[1]) / v.dx[(size_t)v.stride + p[1]] +
-                      (qp[2] * ap[2] - qm[2] * am[2]) / v.dx[2 * (size_t)v.stride + p[2]]) / v.fb[c];
-    return v.Fp[c] - dt * r;
+    w.Fp = v.Fp[c];
+    w.fb = v.fb[c];
 }
-
-__device__ inline double vof_df(const VofDev &v, long c, const int p[3], double dt) {
-    const double z[3] = {0.0, 0.0, 0.0};
-    const bool n[3] = {false, false, false};
-    return vof_df(v, c, p, dt, z, n);
+__device__ __forceinline__ double vof_df(const VofDev &v, const VofCell &w, const int p[3], double dt) {
+    double qp[3], ap[3];
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        qp[l] = w.solid[l] ? 0.0 : w.qh[l];
+        ap[l] = w.solid[l] ? 0.0 : w.ah[l];
+    }
+    const double r = ((qp[0] * ap[0] - w.q[0] * w.a[0]) / v.dx[p[0]] +
+                      (qp[1] * ap[1] - w.q[1] * w.a[1]) / v.dx[(size_t)v.stride + p[1]] +
+                      (qp[2] * ap[2] - w.q[2] * w.a[2]) / v.dx[2 * (size_t)v.stride + p[2]]) / w.fb;
+    return w.Fp - dt * r;
+}
+__device__ __forceinline__ double vof_df(const VofDev &v, long c, const int p[3], double dt, const double sub[3],
+                                         const bool has_sub[3]) {
+    VofCell w;
+    vof_load(v, c, w);
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+        if (has_sub[l]) w.q[l] = w.q[l] - sub[l];
+    return vof_df(v, w, p, dt);
+}
+__device__ __forceinline__ double vof_df(const VofDev &v, long c, const int p[3], double dt) {
+    VofCell w;
+    vof_load(v, c, w);
+    return vof_df(v, w, p, dt);
 }
 
 __device__ inline double vof_sign(double a, double b) { return signbit(b) ? -fabs(a) : fabs(a); }
 
 // MODE 0: caller's PLIC face fluxes where qmask != 0 (qs/qmask may be null);
-// MODE 1: quvwf_kaidan.
+// MODE 1: quvwf_kaidan.  Every load but those of surface donors and partly
+// open faces is issued before the first is used (each waited for the flags
+// it depends on before: 84 us at 4.4M cells, now 58; the fields alone
+// take 51 at a large copy's rate).
 template <int MODE>
 __global__ void __launch_bounds__(256)
-k_vof_flux(VofDev v, double dt, const double *__restrict__ qs, const int8_t *__restrict__ qmask) {
+k_vof_flux(VofDev v, double dt, const double *__restrict__ qs, const int8_t *__restrict__ qmask,
+           const int *__restrict__ cnt) {
     const long c = (long)vof_block() * blockDim.x + threadIdx.x;
     if (c >= v.ncell) return;
     const long st[3] = {1, (long)(v.nx + 2), (long)(v.nx + 2) * (v.ny + 2)};
     const size_t n = (size_t)v.ncell;
-    if (v.nf[c] == -1) {
+    const int fc = v.nf[c], bc = v.nb[c];
+    const double Fc = v.F[c];
+    int fm[3], bm[3];
+    double Fm[3], ul[3], al[3];
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        const long m = max(c - st[l], 0l);  // a ring cell's may lie before the box
+        fm[l] = v.nf[m];
+        bm[l] = v.nb[m];
+        Fm[l] = v.F[m];
+        ul[l] = v.un[l * n + c];
+        al[l] = MODE == 1 && l < 2 ? v.a[l * n + c] : 0.0;
+    }
+    if (!vof_valid(cnt)) return;
+    if (fc == -1) {
+#pragma unroll
         for (int l = 0; l < 3; ++l) v.qf[l * n + c] = 0.0;
         return;
     }
     int p[3];
     vof_pos(v, c, p);
+#pragma unroll
     for (int l = 0; l < 3; ++l) {
         const size_t o = l * n + c;
-        const double u = v.un[o];
+        const double u = ul[l];
         const long m = c - st[l];
         // QFF: the donor is the upwind cell (c - e_l for u > 0, c for u < 0)
         const bool neg = signbit(u);
-        const long nnd = neg ? c : m;
         double q = 0.0;
-        if (u != 0.0 && v.nf[m] != -1) {
-            const int fd = v.nf[nnd], bd = v.nb[nnd];
-            const double Fd = v.F[nnd];
+        if (u != 0.0 && fm[l] != -1) {
+            const int fd = neg ? fc : fm[l], bd = neg ? bc : bm[l];
+            const double Fd = neg ? Fc : Fm[l];
             if (fd == 2 && (bd < 0 ? -bd : bd) == l + 1) {
                 const double dxx = v.dx[(size_t)l * v.stride + (neg ? p[l] : p[l] - 1)];
                 if ((double)bd * u < 0.0) {
@@ -141,13 +193,13 @@ k_vof_flux(VofDev v, double dt, const double *__restrict__ qs, const int8_t *__r
         }
         if (MODE == 1) {
             if (l < 2) {
-                const double av = v.a[o];
+                const double av = al[l];
                 if (av > 0.0 && av < 1.0) {
-                    if (u < 0.0 && v.nf[c] == 2 && av != v.fb[c]) {
-                        const double t = av - v.fb[c] + v.F[c] * v.fb[c];
+                    if (u < 0.0 && fc == 2 && av != v.fb[c]) {
+                        const double t = av - v.fb[c] + Fc * v.fb[c];
                         q = u * (t > 0.0 ? t : 0.0) / av;
-                    } else if (u > 0.0 && v.nf[m] == 2 && av != v.fb[m]) {
-                        const double t = av - v.fb[m] + v.F[m] * v.fb[m];
+                    } else if (u > 0.0 && fm[l] == 2 && av != v.fb[m]) {
+                        const double t = av - v.fb[m] + Fm[l] * v.fb[m];
                         q = u * (t > 0.0 ? t : 0.0) / av;
                     }
                 }
@@ -167,9 +219,10 @@ k_vof_flux(VofDev v, double dt, const double *__restrict__ qs, const int8_t *__r
 // k_vof_flux<0>.  Two listed cells never write one face: the shared face's
 // velocity drains only one of them.
 __global__ void __launch_bounds__(256)
-k_vof_plic(VofDev v, double dt, int n, const int *__restrict__ cells, const double *__restrict__ vol) {
+k_vof_plic(VofDev v, double dt, int n, const int *__restrict__ cells, const double *__restrict__ vol,
+           const int *__restrict__ cnt) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
+    if (m >= n || !vof_valid(cnt)) return;
     const long c = cells[m];
     const long st[3] = {1, (long)(v.nx + 2), (long)(v.nx + 2) * (v.ny + 2)};
     int p[3];
@@ -206,23 +259,66 @@ k_vof_check_plic(VofDev v, int n, const int *__restrict__ cells, int *__restrict
 
 // The flags every other kernel relies on for its neighbour reads: the box
 // ring is solid (nf = -1), nf is -1..2, and a surface cell has 1 <= |nb| <= 3.
-__global__ void __launch_bounds__(256) k_vof_check(VofDev v, int *__restrict__ cnt) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= v.ncell) return;
+// Lists the surface cells, a segment of the list a workgroup, and sets them
+// pending.  Sixteen cells
+// a thread, one load a field where they are aligned (one cell a thread, and a
+// pass that cleared the state of every cell: 14 + 7 us at 4.4M cells; now
+// 13).
+constexpr int VOF_CELLS = 16, VOF_SEG = 64 * VOF_CELLS;  // cells a thread and a list segment
+__global__ void __launch_bounds__(64)
+k_vof_check(VofDev v, int *__restrict__ cnt, int *__restrict__ state, unsigned *__restrict__ list,
+            int *__restrict__ nlist) {
+    const long c0 = VOF_CELLS * ((long)blockIdx.x * blockDim.x + threadIdx.x);
+    int8_t f[VOF_CELLS], b[VOF_CELLS];
+    if (c0 + VOF_CELLS <= v.ncell && (((uintptr_t)v.nf | (uintptr_t)v.nb) & 15) == 0) {
+        *reinterpret_cast<uint4 *>(f) = *reinterpret_cast<const uint4 *>(v.nf + c0);
+        *reinterpret_cast<uint4 *>(b) = *reinterpret_cast<const uint4 *>(v.nb + c0);
+    } else {
+#pragma unroll
+        for (int k = 0; k < VOF_CELLS; ++k) {
+            f[k] = c0 + k < v.ncell ? v.nf[c0 + k] : (int8_t)-1;
+            b[k] = c0 + k < v.ncell ? v.nb[c0 + k] : (int8_t)0;
+        }
+    }
     int p[3];
-    vof_pos(v, c, p);
-    const int f = v.nf[c], b = v.nb[c];
-    const bool ring = p[0] == 0 || p[0] == v.nx + 1 || p[1] == 0 || p[1] == v.ny + 1 || p[2] == 0 || p[2] == v.nz + 1;
-    // object cells of the case (flag -1 with a nonzero object code) are not
-    // covered: QFF's object branches (1sub-vof.F90:77-97) are not restated
-    const bool bad = (ring && f != -1) || f < -1 || f > 2 || (f == 2 && (b == 0 || b < -3 || b > 3)) ||
-                     (f == -1 && b != 0);
+    vof_pos(v, c0, p);
+    bool bad = false;
+    int ns = 0;
+#pragma unroll
+    for (int k = 0; k < VOF_CELLS; ++k) {
+        if (c0 + k < v.ncell) {
+            const bool ring = p[0] == 0 || p[0] == v.nx + 1 || p[1] == 0 || p[1] == v.ny + 1 || p[2] == 0 ||
+                              p[2] == v.nz + 1;
+            // object cells of the case (flag -1 with a nonzero object code) are not
+            // covered: QFF's object branches (1sub-vof.F90:77-97) are not restated
+            bad = bad || (ring && f[k] != -1) || f[k] < -1 || f[k] > 2 ||
+                  (f[k] == 2 && (b[k] == 0 || b[k] < -3 || b[k] > 3)) || (f[k] == -1 && b[k] != 0);
+            if (f[k] == 2) {
+                state[c0 + k] = 0;
+                ++ns;
+            }
+        }
+        if (++p[0] == v.nx + 2) {
+            p[0] = 0;
+            if (++p[1] == v.ny + 2) {
+                p[1] = 0;
+                ++p[2];
+            }
+        }
+    }
     if (bad) atomicOr(&cnt[VC_BAD], 1);
-}
-
-__global__ void __launch_bounds__(256) k_vof_state_init(long n, int *__restrict__ state) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n) state[c] = 0;
+    const int l = threadIdx.x;
+    int at = ns;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(at, d, 64);
+        if (l >= d) at += o;
+    }
+    if (l == 63) nlist[blockIdx.x] = at;
+    unsigned *mine = list + (size_t)blockIdx.x * VOF_SEG + at - ns;
+#pragma unroll
+    for (int k = 0; k < VOF_CELLS; ++k)
+        if (c0 + k < v.ncell && f[k] == 2) *mine++ = (unsigned)(c0 + k);
 }
 
 // state: 0 pending, else 2*round + (1 if the cell's correction term is set).
@@ -230,11 +326,9 @@ __global__ void __launch_bounds__(256) k_vof_state_init(long n, int *__restrict_
 // earlier round (earlier launch), so the term it reads is complete.
 __device__ inline bool vof_decided(int s, int round) { return s != 0 && (s >> 1) < round; }
 
-__global__ void __launch_bounds__(256)
-k_vof_mod_eval(VofDev v, double dt, int round, int *__restrict__ state, double *__restrict__ term,
-               int *__restrict__ cnt) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= v.ncell || v.nf[c] != 2 || state[c] != 0) return;
+__device__ __forceinline__ void vof_mod_cell(const VofDev &v, double dt, int round, int *state, double *term, long c,
+                                             int *cnt, int slot) {
+    if (state[c] != 0) return;
     const long st[3] = {1, (long)(v.nx + 2), (long)(v.nx + 2) * (v.ny + 2)};
     double sub[3] = {0.0, 0.0, 0.0};
     bool has[3] = {false, false, false};
@@ -243,7 +337,7 @@ k_vof_mod_eval(VofDev v, double dt, int round, int *__restrict__ state, double *
         if (v.nf[r] == 2 && v.nb[r] == -(l + 1)) {
             const int s = state[r];
             if (!vof_decided(s, round)) {
-                atomicAdd(&cnt[VC_PENDING], 1);
+                atomicAdd(&cnt[slot], 1);
                 return;
             }
             if (s & 1) {
@@ -268,10 +362,20 @@ k_vof_mod_eval(VofDev v, double dt, int round, int *__restrict__ state, double *
     atomicAdd(&cnt[VC_MODIFIED], 1);
 }
 
+// One round over the listed cells (a workgroup a segment), pending cells
+// counted at cnt[slot]; not run where the round before (counted at prev, < 0:
+// none) left none.
 __global__ void __launch_bounds__(256)
-k_vof_mod_apply(VofDev v, const int *__restrict__ state, const double *__restrict__ term) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= v.ncell || v.nf[c] != 2 || !(state[c] & 1)) return;
+k_vof_mod_eval(VofDev v, double dt, int round, int *__restrict__ state, double *__restrict__ term,
+               const unsigned *__restrict__ list, const int *__restrict__ nlist, int *cnt, int prev, int slot) {
+    if (!vof_valid(cnt) || (prev >= 0 && cnt[prev] == 0)) return;
+    const int n = nlist[blockIdx.x];
+    const unsigned *mine = list + (size_t)blockIdx.x * VOF_SEG;
+    for (int q = threadIdx.x; q < n; q += 256) vof_mod_cell(v, dt, round, state, term, (long)mine[q], cnt, slot);
+}
+
+__device__ __forceinline__ void vof_apply_cell(const VofDev &v, const int *state, const double *term, long c) {
+    if (!(state[c] & 1)) return;
     const long st[3] = {1, (long)(v.nx + 2), (long)(v.nx + 2) * (v.ny + 2)};
     const int b = v.nb[c], l = (b < 0 ? -b : b) - 1;
     const size_t n = (size_t)v.ncell;
@@ -288,20 +392,35 @@ k_vof_mod_apply(VofDev v, const int *__restrict__ state, const double *__restric
         v.qf[l * n + t] = v.qf[l * n + t] - term[c];
     }
 }
+// Runs once no cell is pending; the last queued round's count becomes
+// VC_PENDING's.
+__global__ void __launch_bounds__(256)
+k_vof_mod_apply(VofDev v, const int *__restrict__ state, const double *__restrict__ term,
+                const unsigned *__restrict__ list, const int *__restrict__ nlist, const int *cnt) {
+    if (!vof_settled(cnt)) return;
+    const int n = nlist[blockIdx.x];
+    const unsigned *mine = list + (size_t)blockIdx.x * VOF_SEG;
+    for (int q = threadIdx.x; q < n; q += 256) vof_apply_cell(v, state, term, (long)mine[q]);
+}
 
-__global__ void __launch_bounds__(256) k_vof_newf(VofDev v, double dt, int *__restrict__ cnt) {
+// What bounds it is HBM: 80 bytes a cell (waiting for the flags before the
+// faces: 78 us at 4.4M cells; now 75, 57 at a large copy's rate).
+__global__ void __launch_bounds__(256) k_vof_newf(VofDev v, double dt, int *cnt) {
     const long c = (long)vof_block() * blockDim.x + threadIdx.x;
     if (c >= v.ncell) return;
     const int f = v.nf[c];
+    VofCell w;
+    vof_load(v, c, w);
+    if (!vof_settled(cnt)) return;
     if (f == -1) {
         v.Fn[c] = v.F[c];
         return;
     }
     int p[3];
     vof_pos(v, c, p);
-    double d = vof_df(v, c, p, dt);
+    double d = vof_df(v, w, p, dt);
     v.D[c] = d;
-    if (-d * dt * v.fb[c] > 0.4) {
+    if (-d * dt * w.fb > 0.4) {
         atomicOr(&cnt[VC_RETRY], 1);
     } else if (fabs(d * dt) < VOF_TINY && d != 0.0) {
         d = 0.0;
@@ -316,9 +435,20 @@ __global__ void __launch_bounds__(256) k_vof_newf(VofDev v, double dt, int *__re
 // this column changed a face since: the cell's high face is changed by a
 // move one level up (then its df_vof is the value that move left for the
 // cell below), the lower cell's faces only by moves not yet made.
-__global__ void __launch_bounds__(256) k_vof_slide(VofDev v, double dt, int *__restrict__ cnt) {
+//
+// A column is a serial walk of nz levels and there are only nx ny of them, so
+// what bounds this is the chain of loads.  The flags of VOF_LEVELS levels are
+// loaded at once, ahead of the walk, and where one of them may slide so are
+// their D and fb; a move takes one trip more.  At 256 x 256 columns of 64 of
+// which 25 levels slide, 76 us (one load after the other, and one counter for
+// all moves: 144).  Everything a move needs loaded ahead: 72 to 77, and more
+// where nothing slides; columns in 8 x 8 or 16 x 4 tiles: 80 to 88; 32 columns a
+// wavefront: 96.
+constexpr int VOF_LEVELS = 8;
+__global__ void __launch_bounds__(64) k_vof_slide(VofDev v, double dt, int *cnt) {
     const int col = vof_block() * blockDim.x + threadIdx.x;
     if (col >= v.nx * v.ny) return;
+    if (!vof_settled(cnt) || (cnt[VC_RETRY] | cnt[VC_STOP]) != 0) return;
     const int i = 1 + col % v.nx, j = 1 + col / v.nx;
     const long X = v.nx + 2, Y = v.ny + 2, sz = X * Y;
     const size_t S = (size_t)v.stride;
@@ -326,42 +456,71 @@ __global__ void __launch_bounds__(256) k_vof_slide(VofDev v, double dt, int *__r
     int moved = 0;
     bool changed_above = false;  // qf(2, c + e_z) moved by the previous level
     double carried = 0.0;        // df_vof(c) after that move
-    for (int k = v.nz; k >= 1; --k) {
-        const long c = i + X * (j + Y * k), m = c - sz;
-        const int f = v.nf[c];
-        if (f == -1) break;
-        if (f == 1 || v.nf[m] == -1) {
-            changed_above = false;
-            continue;
+    const long c0 = i + X * j;
+    bool open = true;            // no solid cell met
+    int nf[VOF_LEVELS + 1];      // of levels k0 .. k0 - VOF_LEVELS (level 0, solid, below them)
+#pragma unroll
+    for (int u = 0; u <= VOF_LEVELS; ++u) nf[u] = v.nf[c0 + sz * max(v.nz - u, 0)];
+    for (int k0 = v.nz; k0 >= 1 && open; k0 -= VOF_LEVELS) {
+        int nx[VOF_LEVELS + 1];  // the next levels'
+#pragma unroll
+        for (int u = 0; u <= VOF_LEVELS; ++u) nx[u] = v.nf[c0 + sz * max(k0 - VOF_LEVELS - u, 0)];
+        bool any = false;
+#pragma unroll
+        for (int u = 0; u < VOF_LEVELS; ++u) any = any || (nf[u] != 1 && nf[u] != -1);
+        double fb[VOF_LEVELS + 1], D[VOF_LEVELS + 1], dz[VOF_LEVELS + 1];
+        if (any) {
+#pragma unroll
+            for (int u = 0; u <= VOF_LEVELS; ++u) {
+                const int k = max(k0 - u, 0);
+                fb[u] = v.fb[c0 + sz * k];
+                D[u] = v.D[c0 + sz * k];  // of a solid cell: not used
+                dz[u] = v.dx[2 * S + k];
+            }
         }
-        const double vmesh = dx0 * dx1 * v.dx[2 * S + k];
-        const double dvc = vmesh * v.fb[c];
-        const double dvm = dx0 * dx1 * v.dx[2 * S + k - 1] * v.fb[m];
-        if (dvc * dvm == 0.0) {
+#pragma unroll
+        for (int u = 0; u < VOF_LEVELS; ++u) {
+            const int k = k0 - u;
+            if (!open || k < 1) continue;
+            const long c = c0 + sz * k, m = c - sz;
+            if (nf[u] == -1) {
+                open = false;
+                continue;
+            }
+            const bool above = changed_above;
             changed_above = false;
-            continue;
+            if (nf[u] == 1 || nf[u + 1] == -1) continue;
+            const double vmesh = dx0 * dx1 * dz[u];
+            const double dvc = vmesh * fb[u];
+            const double dvm = dx0 * dx1 * dz[u + 1] * fb[u + 1];
+            if (dvc * dvm == 0.0) continue;
+            const double fc = above ? carried : D[u];
+            const double fm = D[u + 1];
+            v.Fn[c] = fc;
+            v.Fn[m] = fm;
+            const double t1 = dvm * (1.0 - fm), t2 = dvc * fc;
+            const double f2 = t1 < t2 ? t1 : t2;
+            if (fabs(f2) == 0.0) continue;
+            // both cells' fields before the move, in one trip; the moved face is
+            // the one's low and the other's high
+            VofCell wc, wm;
+            vof_load(v, c, wc);
+            vof_load(v, m, wm);
+            const double q = wc.q[2] + -1.0 * f2 / vmesh / dt * dz[u] / wc.a[2];
+            v.qf[2 * (size_t)v.ncell + c] = q;
+            wc.q[2] = wm.qh[2] = q;
+            const int pc[3] = {i, j, k}, pm[3] = {i, j, k - 1};
+            const double ft = vof_df(v, wc, pc, dt);
+            v.Fn[c] = fabs(ft) < VOF_TINY ? 0.0 : ft;
+            carried = vof_df(v, wm, pm, dt);
+            v.Fn[m] = carried;
+            changed_above = true;
+            ++moved;
         }
-        const double fc = changed_above ? carried : v.D[c];
-        const double fm = v.D[m];
-        v.Fn[c] = fc;
-        v.Fn[m] = fm;
-        const double t1 = dvm * (1.0 - fm), t2 = dvc * fc;
-        const double f2 = t1 < t2 ? t1 : t2;
-        if (fabs(f2) == 0.0) {
-            changed_above = false;
-            continue;
-        }
-        const size_t o = 2 * (size_t)v.ncell + c;
-        v.qf[o] = v.qf[o] + -1.0 * f2 / vmesh / dt * v.dx[2 * S + k] / v.a[o];
-        const int pc[3] = {i, j, k}, pm[3] = {i, j, k - 1};
-        const double ft = vof_df(v, c, pc, dt);
-        v.Fn[c] = fabs(ft) < VOF_TINY ? 0.0 : ft;
-        carried = vof_df(v, m, pm, dt);
-        v.Fn[m] = carried;
-        changed_above = true;
-        ++moved;
+#pragma unroll
+        for (int u = 0; u <= VOF_LEVELS; ++u) nf[u] = nx[u];
     }
-    if (moved) atomicAdd(&cnt[VC_SLID], moved);
+    if (moved) atomicAdd(&cnt[VC_SLID + VC_LINE * (blockIdx.x % VC_SLOTS)], moved);
 }
 
 } // namespace clowns

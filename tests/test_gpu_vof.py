@@ -167,3 +167,53 @@ def test_vof_plic_rejects_solid_cell():
         dg.vof(sol, Fp, dt=dt, plic=(cells, vol))
     assert e.value.code == CLOWNS_EBADARG
     sol.close()
+
+
+@pytest.mark.parametrize("length", [1, 2, 3, 4, 5])
+def test_vof_chain_lengths_around_the_queued_rounds(length):
+    """The first rounds of quvwf_modify are queued with everything after them,
+    which stands back while cells are pending: chains shorter and longer than
+    those rounds."""
+    from clowns3d import assembly
+    g, A, Fp, dt = vof_case("wavy20x16x12", "step", seed=9)
+    c = assembly.classify(g)
+    nf, nb = c["nf"].copy(), c["nb"].copy()
+    stack = [5 + g.X * (6 + g.Y * k) for k in range(2, 2 + length)]
+    for q in stack:
+        assert c["arrays"]["solid"][q] == 0
+        nf[q], nb[q] = 2, -3
+    c = dict(c, nf=nf, nb=nb)
+    Fp = Fp.copy()
+    Fp[stack] = 1.0 + 1e-3
+    o, info = compare(g, c, Fp, dt, 1)
+    assert o["modified"] >= length and info["rounds"] >= length
+
+
+@pytest.mark.parametrize("shape", [(9, 7, 5), (17, 5, 8), (13, 11, 9), (63, 3, 7), (31, 33, 17)])
+def test_vof_odd_boxes_and_unaligned_flags(shape):
+    """Boxes whose columns, levels and cells leave remainders in every kernel,
+    with fluid, air and noise in every cell (each level may slide), and flags
+    that start at an odd byte."""
+    import torch
+    from clowns3d import DeviceGrid, Solver, assembly, configs
+    nx, ny, nz = shape
+    g = configs.config_wavy_box(nx, ny, nz, (1, 3, 1, 2, 0, 2))
+    rng = np.random.default_rng(nx)
+    g.un[:] = rng.uniform(-0.1, 0.1, size=g.un.shape)
+    c = assembly.classify(g)
+    Fp = np.clip(c["F"] + rng.uniform(-0.01, 0.01, size=c["F"].shape), 0.0, 1.0)
+    Fp[c["arrays"]["solid"] != 0] = 0.0
+    o, info = compare(g, c, Fp, g.dt, 1)
+    assert o["slid"] > 0
+    sol = Solver(0)
+    dg = DeviceGrid(g, classified=c)
+    keep = []
+    for name in ("nf", "nb"):  # the device view's pointers, at odd addresses
+        t = dg.t[name].view(-1)
+        keep.append(torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].copy_(t))
+        assert keep[-1].data_ptr() % 2 == 1
+        setattr(dg.dev, name, keep[-1].data_ptr())
+    Fn, qf, info2 = dg.vof(sol, Fp, mode=1, dt=g.dt)
+    assert np.array_equal(Fn.cpu().numpy(), o["F"]) and np.array_equal(qf.cpu().numpy(), o["qf"])
+    assert {k: info2[k] for k in ("modified", "slid", "rounds")} == {k: info[k] for k in ("modified", "slid", "rounds")}
+    sol.close()
