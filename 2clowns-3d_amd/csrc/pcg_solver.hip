@@ -1613,7 +1613,7 @@ int assign_patterns(clowns_solver *h, int *nnone) {
     const int N = h->N;
     fill<int>(s, h->flag.p, 2, 0);
     const int npad = n_pad(N) + 4;
-    k_pat_assign<<<cdiv(npad, BS), BS, 0, s>>>(N, npad, h->lda, h->AL.p, h->D.p, h->LL.p, h->ptab.p, h->npat,
+    k_pat_assign<<<cdiv(npad, BS * PAT_PER), BS, 0, s>>>(N, npad, h->lda, h->AL.p, h->D.p, h->LL.p, h->ptab.p, h->npat,
                                                h->pid.p, h->flag.p);
     HIPCHK(hipGetLastError());
     int res[2] = {0, 0};
@@ -1676,6 +1676,14 @@ int build_patterns(clowns_solver *h) {
     return CLOWNS_OK;
 }
 
+// The blocks' places among the packed tasks in a block order (null: natural).
+void scan_runs(clowns_solver *h, const int *order) {
+    const int nblk = cdiv(h->N, RUN_ROWS), G = geo_of(h->N, 2).G;
+    int *pos = h->run_n.p + 2 * nblk;
+    k_run_counts<<<cdiv(G, BS), BS, 0, h->stream>>>(G, nblk, order, h->run_n.p, h->run_n.p + nblk, pos);
+    k_cls_scan_blocks<<<1, 1024, 0, h->stream>>>(G, pos);
+    k_cls_scan_blocks<<<1, 1024, 0, h->stream>>>(G, pos + G + 1);
+}
 // The packed tasks of one precision in a block order (null: natural).
 template <typename T, typename C>
 int pack_runs(clowns_solver *h, const int *order, DevBuf<RunPair<T>> *pair, DevBuf<RunSpmv<T>> &sp,
@@ -1689,9 +1697,7 @@ int pack_runs(clowns_solver *h, const int *order, DevBuf<RunPair<T>> *pair, DevB
     hipStream_t s = h->stream;
     const int *n0 = h->run_n.p, *n1 = n0 + nblk;
     int *pos = h->run_n.p + 2 * nblk;
-    k_run_counts<<<cdiv(G, BS), BS, 0, s>>>(G, nblk, order, n0, n1, pos);
-    k_cls_scan_blocks<<<1, 1024, 0, s>>>(G, pos);
-    k_cls_scan_blocks<<<1, 1024, 0, s>>>(G, pos + G + 1);
+    scan_runs(h, order);
     k_run_pack<T, C><<<cdiv((long)G * RUN_TASKS, BS), BS, 0, s>>>(G, nblk, order, n0, n1, pos, h->run_raw[0].p,
                                                                  h->run_raw[1].p, h->run_raws.p, pair[0].p,
                                                                  pair[1].p, sp.p);
@@ -1746,7 +1752,11 @@ int build_runs(clowns_solver *h) {
     o.rc = h->run_rc.p;
     o.lcap = lcap;
     o.rcap = rcap;
-    k_run_build<<<nblk, BS, 0, s>>>(N, h->lda, h->AL.p, h->D.p, h->LL.p, h->pid.p, o, h->flag.p);
+    // flag: list entries and records, then the tasks of both kinds
+    k_run_build<<<nblk, BS, 0, s>>>(N, h->lda, h->AL.p, h->D.p, h->LL.p, h->pid.p, o,
+                                    reinterpret_cast<unsigned long long *>(h->flag.p));
+    scan_runs(h, nullptr);
+    k_run_totals<<<1, 64, 0, s>>>(G, h->run_n.p + 2 * nblk, h->flag.p + 2);
     HIPCHK(hipGetLastError());
     int res[4] = {0, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(res, h->flag.p, 4 * sizeof(int), hipMemcpyDeviceToHost, s));

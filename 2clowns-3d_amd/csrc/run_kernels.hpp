@@ -133,11 +133,12 @@ __device__ __forceinline__ void run_bounds(const unsigned long long *heads, int 
 // one pattern (the row's and its partners'), then, over what is left, those of
 // any coefficients (RF_OWN).  List entries and records come from an atomic
 // allocation (their place depends on the run, their contents do not; past lcap
-// and rcap none are written).  cnt: list entries, records, table tasks, own
-// tasks.
+// and rcap none are written).  cnt: list entries, records << 32: one atomic a
+// block (the four counters of a first form, of which atomics on one address
+// are some 6 ns each, were its time: 613 us at 6.6M rows, now 224).
 __global__ void __launch_bounds__(BS)
 k_run_build(int N, int lda, const double *__restrict__ AL, const double *__restrict__ D, const int *__restrict__ LL,
-            const uint8_t *__restrict__ pid, RunBuild o, int *__restrict__ cnt) {
+            const uint8_t *__restrict__ pid, RunBuild o, unsigned long long *__restrict__ cnt) {
     const int r0 = blockIdx.x * RUN_ROWS, t = threadIdx.x;
     constexpr int KW = 9;  // six offsets, the partners' two, patterns
     __shared__ int key[KW][RUN_ROWS];
@@ -258,12 +259,11 @@ k_run_build(int N, int lda, const double *__restrict__ AL, const double *__restr
     const unsigned tot = pre[RUN_ROWS - 1];
     if (t == 0) {
         const int nl = tot & 1023, nr = tot >> 10 & 1023;
-        start[0] = nl ? atomicAdd(&cnt[0], nl) : 0;
-        start[1] = nr ? atomicAdd(&cnt[1], nr) : 0;
+        const unsigned long long at = nl | nr ? atomicAdd(cnt, (unsigned long long)nr << 32 | nl) : 0;
+        start[0] = (int)(unsigned)at;
+        start[1] = (int)(at >> 32);
         o.nt0[blockIdx.x] = tot >> 20 & 63;
         o.nt1[blockIdx.x] = tot >> 26;
-        atomicAdd(&cnt[2], tot >> 20 & 63);
-        atomicAdd(&cnt[3], tot >> 26);
     }
     __syncthreads();
     if (o.cid && t < 4) {
@@ -353,6 +353,10 @@ k_run_counts(int G, int nblk, const int *__restrict__ order, const int *__restri
     const int rb = order ? order[i] : i;
     out[i] = rb < nblk ? nt0[rb] : 0;
     out[G + 1 + i] = rb < nblk ? nt1[rb] : 0;
+}
+// Tasks of both kinds from the scanned counts.
+__global__ void k_run_totals(int G, const int *__restrict__ pos, int *__restrict__ out) {
+    if (threadIdx.x < 2) out[threadIdx.x] = pos[threadIdx.x ? 2 * G + 1 : G];
 }
 // The wavefronts of k_pm_dot_run (R rows a lane) in launch order.
 template <int R>
