@@ -399,7 +399,7 @@ struct clowns_solver {
     // per time step at 26M rows; 2e-2 .. 1e-1 and 3e-4 were slower.
     double tau_min = 1e-2;
     bool cls_force_host = false;  // test hook: always take the exact host path
-    int poll = 3;          // iterations queued ahead of the last one seen done
+    int poll = 4;          // iterations queued ahead of the last one seen done, at the least
     int will_max_rounds = 4096;  // PCGPME_WILL output pass: device rounds before the host pass
     int fuse64 = -1, fuse32 = -1;      // pairwise PM fusion chosen by tune_fuse ...
     int fuse64_N = 0, fuse32_N = 0;    // ... for operators of about this many rows (tuned_size)
@@ -1022,12 +1022,15 @@ template <typename T> void known_stream(const clowns_solver *h, Op<T> &A) {
     if (!A.run.spmv && stored_forms(h, A, &f)) set_forms(A, f);
 }
 
+constexpr int QUEUE_MAX = 16;  // iterations a run queues ahead at the most (and h->poll at the least)
+
 // The PCGPME iteration (pcgpme_para.F90:148-247) on already initialised
 // vectors: V.p0 = V.r = V.rh = r0, V.x = x0, scalars BN/C1 set by k_fin_init,
 // h->run_word cleared before that.  Returns with the stream drained after the
 // device has set `done`; the final scalars are in h->h_sc[sc_index].
 template <typename T>
-int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int itermax, int sc_index) {
+int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int itermax, int sc_index,
+                 double eps) {
     hipStream_t s = h->stream;
     double *part = h->part.p;
     const int Gv = geo_of(A.N, VecOf<T>::R).G;
@@ -1116,15 +1119,19 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
     // and posts the iterations done and the decision to a word of host memory,
     // in the next iteration's first kernel (at the end of k_fin_beta, whose own
     // end then waits for the host's memory, it cost 2 us an iteration).
-    // The host queues h->poll iterations ahead of the last one it saw there:
-    // enough that the GPU never waits for it, and few to run out at the end.
+    // The host queues up to QUEUE_MAX iterations ahead of the last one it saw
+    // there, so that a host held up for a millisecond leaves the GPU work, but
+    // h->poll near the end, which it predicts from ERR at the last words
+    // (Bi-CGSTAB converges about geometrically): few then run out for nothing.
     int K = 1, seen = 0;
     const int last = itermax + 1;  // whose first kernel posts the last iteration's word
     bool done = itermax <= 0;  // PCGPME_WILL may ask for none
-    int spins = 0;
+    int spins = 0, ahead = std::max(h->poll, QUEUE_MAX / 2);
+    int kp = 0;        // an earlier word's iterations and ERR
+    double ep = 0.0;
     while (!done) {
         const int k0 = K;
-        while (K <= last && K - 1 - seen < h->poll) iteration(K++);
+        while (K <= last && K - 1 - seen < ahead) iteration(K++);
         if (K != k0) HIPCHK(hipGetLastError());
         const unsigned long long w = __atomic_load_n(host, __ATOMIC_RELAXED);
         const int k = (int)(w >> 33);
@@ -1132,6 +1139,21 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
         if (done || k != seen) {
             seen = k;
             spins = 0;
+            if (k - kp >= 4) {
+                const unsigned bits = (unsigned)w;
+                float ef;
+                std::memcpy(&ef, &bits, sizeof(ef));
+                const double e = ef, rate = kp > 0 ? std::log(ep / e) / (k - kp) : 0.0;
+                if (rate > 0.0 && eps > 0.0) {
+                    const double left = std::log(e / eps) / rate;  // iterations to go
+                    ahead = !(left < QUEUE_MAX) ? QUEUE_MAX : (int)std::max(left, 0.0);
+                }
+                ahead = std::max(h->poll, ahead);
+                kp = k;
+                ep = e;
+            } else if (ahead > h->poll) {
+                --ahead;  // as the predicted end comes nearer
+            }
             continue;
         }
         if (++spins < 20000) {
@@ -1158,7 +1180,6 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
 
 int check_nl(int NL) { return (NL == 6 || NL == 4) ? CLOWNS_OK : CLOWNS_EBADNL; }
 
-int build_ll8(clowns_solver *h);
 int build_forms(clowns_solver *h);
 int build_runs32(clowns_solver *h);
 int order_runs(clowns_solver *h);
@@ -1586,52 +1607,37 @@ int ensure_f32(clowns_solver *h) {
 // The 16-bit form of the resident sorted LL, used by the two-row kernels
 // when every offset fits (always, for box grids up to 16383 cells a line).
 int build_ll16(clowns_solver *h) {
-    h->ll16_ok = false;
-    h->ll16_wide = 0;
+    h->ll16_ok = h->ll8_ok = false;
+    h->ll16_wide = h->ll8_wide = 0;
     if (!h->kn.ll16) return CLOWNS_OK;
-    const int N = h->N, nblk = cdiv(N, LL16_ROWS);
+    const int N = h->N, nblk = cdiv(N, LL16_ROWS), nblk8 = cdiv(N, LL8_ROWS);
+    const size_t nm = (size_t)h->lda * h->NL;
+    // the 8-bit codes are not needed where both precisions were timed at this
+    // size and kept the 16-bit ones: an assembly per time step need not rebuild
+    // them
+    const bool k64 = h->ix64 == 0 && tuned_size(h->N, h->ix64_N) && h->st64_f == force_key(h);
+    const bool k32 = h->ix32 == 0 && tuned_size(h->N, h->ix32_N) && h->st32_f == force_key(h);
+    const bool want8 = h->kn.ll8 != 0 && !(h->kn.ll8 < 0 && k64 && k32);
     int rc;
-    if ((rc = h->LL16.ensure((size_t)h->lda * h->NL)) || (rc = h->base16.ensure(nblk)) || (rc = h->flag.ensure(2)))
-        return rc;
+    if ((rc = h->LL16.ensure(nm)) || (rc = h->base16.ensure(nblk)) || (rc = h->flag.ensure(4))) return rc;
+    if (want8 && ((rc = h->LL8.ensure(nm)) || (rc = h->base8.ensure(nblk8)))) return rc;
     hipStream_t s = h->stream;
-    fill<int>(s, h->flag.p, 2, 0);
+    fill<int>(s, h->flag.p, 4, 0);
     k_ll16_build<<<nblk, BS, 0, s>>>(N, h->lda, h->NL, h->LL.p, h->LL16.p, h->base16.p, h->flag.p,
                                      h->flag.p + 1);
+    if (want8)
+        k_ll8_build<<<nblk8, BS, 0, s>>>(N, h->lda, h->NL, h->LL.p, h->LL8.p, h->base8.p, h->flag.p + 2,
+                                         h->flag.p + 3);
     HIPCHK(hipGetLastError());
-    int res[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(res, h->flag.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    int res[4] = {0, 0, 0, 0};
+    HIPCHK(hipMemcpyAsync(res, h->flag.p, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     h->ll16_ok = res[0] == 0;
     h->ll16_wide = res[1];
-    return build_ll8(h);
-}
-
-// The 8-bit form (Ix8), built beside the 16-bit one (which stays the
-// fallback: CLOWNS_LL8 = 0).
-int build_ll8(clowns_solver *h) {
-    h->ll8_ok = false;
-    h->ll8_wide = 0;
-    if (h->kn.ll8 == 0 || !h->ll16_ok) return CLOWNS_OK;
-    // not needed where both precisions were timed at this size and kept the
-    // 16-bit codes: an assembly per time step need not rebuild them
-    const bool k64 = h->ix64 == 0 && tuned_size(h->N, h->ix64_N) && h->st64_f == force_key(h);
-    const bool k32 = h->ix32 == 0 && tuned_size(h->N, h->ix32_N) && h->st32_f == force_key(h);
-    if (h->kn.ll8 < 0 && k64 && k32) return CLOWNS_OK;
-    const int N = h->N, nblk = cdiv(N, LL8_ROWS);
-    int rc;
-    if ((rc = h->LL8.ensure((size_t)h->lda * h->NL)) || (rc = h->base8.ensure(nblk)) || (rc = h->flag.ensure(2)))
-        return rc;
-    hipStream_t s = h->stream;
-    fill<int>(s, h->flag.p, 2, 0);
-    k_ll8_build<<<nblk, BS, 0, s>>>(N, h->lda, h->NL, h->LL.p, h->LL8.p, h->base8.p, h->flag.p, h->flag.p + 1);
-    HIPCHK(hipGetLastError());
-    int res[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(res, h->flag.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    h->ll8_ok = res[0] == 0;
-    h->ll8_wide = res[1];
-    if (h->kn.verbose)
-        fprintf(stderr, "clowns_pcg: N=%d 8-bit neighbour codes: %d of %d slots wide\n", N, res[1], N * h->NL);
+    h->ll8_ok = want8 && h->ll16_ok && res[2] == 0;
+    h->ll8_wide = want8 ? res[3] : 0;
+    if (h->kn.verbose && want8)
+        fprintf(stderr, "clowns_pcg: N=%d 8-bit neighbour codes: %d of %d slots wide\n", N, res[3], N * h->NL);
     return CLOWNS_OK;
 }
 
@@ -2043,7 +2049,7 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
     k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1, h->run_word());
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(h->ev2, s));
-    if ((rc = run_bicgstab<double>(h, A, V, sc, itermax, 0))) return rc;
+    if ((rc = run_bicgstab<double>(h, A, V, sc, itermax, 0, eps))) return rc;
     HIPCHK(hipMemcpyAsync(d_x, V.x.p, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, s));
     HIPCHK(hipEventRecord(h->ev1, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -2139,7 +2145,7 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
             k_init<float><<<G1, BS, 0, s>>>(sc, N, F.p0.p, nullptr, F.r.p, F.rh.p, part);
             *h->run_word() = 0;
             k_fin_init<<<1, FIN_BS, 0, s>>>(sc, part, G1, h->run_word());
-            if ((rc = run_bicgstab<float>(h, A32, F, sc, std::max(1, itermax - total_inner), 0)))
+            if ((rc = run_bicgstab<float>(h, A32, F, sc, std::max(1, itermax - total_inner), 0, tau)))
                 return rc;
             total_inner += std::max(0, std::min(h->h_sc[0].kout, itermax));
             ++refinements;
@@ -2833,7 +2839,7 @@ extern "C" int clowns_solver_time_kernel(clowns_solver *h, int32_t kernel, int32
 
 namespace {
 // The 16- and 8-bit codes of the transposed operator's sorted LL, as
-// build_ll16 / build_ll8 make them for the forward one.
+// build_ll16 makes them for the forward one.
 int build_codes_t(clowns_solver *h) {
     h->t16_ok = h->t8_ok = false;
     if (!h->kn.ll16) return CLOWNS_OK;
