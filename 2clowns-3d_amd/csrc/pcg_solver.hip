@@ -399,7 +399,7 @@ struct clowns_solver {
     // per time step at 26M rows; 2e-2 .. 1e-1 and 3e-4 were slower.
     double tau_min = 1e-2;
     bool cls_force_host = false;  // test hook: always take the exact host path
-    int poll = 4;          // iterations queued ahead of the last one seen done, at the least
+    int poll = 3;          // iterations queued ahead of the last one seen done, at the least
     int will_max_rounds = 4096;  // PCGPME_WILL output pass: device rounds before the host pass
     int fuse64 = -1, fuse32 = -1;      // pairwise PM fusion chosen by tune_fuse ...
     int fuse64_N = 0, fuse32_N = 0;    // ... for operators of about this many rows (tuned_size)
@@ -1121,14 +1121,14 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
     // end then waits for the host's memory, it cost 2 us an iteration).
     // The host queues up to QUEUE_MAX iterations ahead of the last one it saw
     // there, so that a host held up for a millisecond leaves the GPU work, but
-    // h->poll near the end, which it predicts from ERR at the last words
-    // (Bi-CGSTAB converges about geometrically): few then run out for nothing.
+    // only a quarter of those to go by the mean rate so far (Bi-CGSTAB converges
+    // about geometrically), and h->poll at the least: the ones queued past the
+    // end run out for nothing, which 8 to 16 at the end of each inner solve of a
+    // mixed one made 4% of a time step.
     int K = 1, seen = 0;
     const int last = itermax + 1;  // whose first kernel posts the last iteration's word
     bool done = itermax <= 0;  // PCGPME_WILL may ask for none
-    int spins = 0, ahead = std::max(h->poll, QUEUE_MAX / 2);
-    int kp = 0;        // an earlier word's iterations and ERR
-    double ep = 0.0;
+    int spins = 0, ahead = h->poll;
     while (!done) {
         const int k0 = K;
         while (K <= last && K - 1 - seen < ahead) iteration(K++);
@@ -1139,21 +1139,12 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
         if (done || k != seen) {
             seen = k;
             spins = 0;
-            if (k - kp >= 4) {
-                const unsigned bits = (unsigned)w;
-                float ef;
-                std::memcpy(&ef, &bits, sizeof(ef));
-                const double e = ef, rate = kp > 0 ? std::log(ep / e) / (k - kp) : 0.0;
-                if (rate > 0.0 && eps > 0.0) {
-                    const double left = std::log(e / eps) / rate;  // iterations to go
-                    ahead = !(left < QUEUE_MAX) ? QUEUE_MAX : (int)std::max(left, 0.0);
-                }
-                ahead = std::max(h->poll, ahead);
-                kp = k;
-                ep = e;
-            } else if (ahead > h->poll) {
-                --ahead;  // as the predicted end comes nearer
-            }
+            const unsigned bits = (unsigned)w;
+            float e;
+            std::memcpy(&e, &bits, sizeof(e));
+            const double rate = k > 0 ? -std::log((double)e) / k : 0.0;  // ERR starts at 1
+            const double left = rate > 0.0 && eps > 0.0 ? std::log(e / eps) / rate : 0.0;  // iterations to go
+            ahead = left > 4.0 * QUEUE_MAX ? QUEUE_MAX : std::max(h->poll, left > 0.0 ? (int)(left / 4.0) : 0);
             continue;
         }
         if (++spins < 20000) {
