@@ -282,6 +282,11 @@ struct Knobs {
 // stands in for the launches costs more than they do.
 template <typename T> constexpr int SMALL_ROWS = sizeof(T) == 8 ? 120000 : 300000;
 template <typename T> constexpr int FUSED_ROWS = sizeof(T) == 8 ? 360000 : 700000;
+// Iterations a run queues ahead of the last one the host has seen done: at the
+// most, and the least that h->poll may ask for (one iteration's word is posted
+// by the next one's first kernel: with none queued behind it the host would
+// wait for a word that no kernel posts).
+constexpr int QUEUE_MAX = 16, QUEUE_MIN = 2;
 
 struct clowns_solver {
     Knobs kn;
@@ -399,7 +404,7 @@ struct clowns_solver {
     // per time step at 26M rows; 2e-2 .. 1e-1 and 3e-4 were slower.
     double tau_min = 1e-2;
     bool cls_force_host = false;  // test hook: always take the exact host path
-    int poll = 3;          // iterations queued ahead of the last one seen done, at the least
+    int poll = 3;          // iterations queued ahead of the last one seen done, at the least (QUEUE_MIN .. QUEUE_MAX)
     int will_max_rounds = 4096;  // PCGPME_WILL output pass: device rounds before the host pass
     int fuse64 = -1, fuse32 = -1;      // pairwise PM fusion chosen by tune_fuse ...
     int fuse64_N = 0, fuse32_N = 0;    // ... for operators of about this many rows (tuned_size)
@@ -1022,7 +1027,6 @@ template <typename T> void known_stream(const clowns_solver *h, Op<T> &A) {
     if (!A.run.spmv && stored_forms(h, A, &f)) set_forms(A, f);
 }
 
-constexpr int QUEUE_MAX = 16;  // iterations a run queues ahead at the most (and h->poll at the least)
 
 // The PCGPME iteration (pcgpme_para.F90:148-247) on already initialised
 // vectors: V.p0 = V.r = V.rh = r0, V.x = x0, scalars BN/C1 set by k_fin_init,
@@ -1155,9 +1159,11 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
         const hipError_t q = hipStreamQuery(s);
         if (q == hipErrorNotReady) continue;
         HIPCHK(q);
-        // the queue ran dry: the word was posted before that
+        // The queue ran dry: a word was posted before that, since at least
+        // QUEUE_MIN iterations were queued past `seen` or the one past itermax
+        // was (by which the device has set done).
         const unsigned long long w2 = __atomic_load_n(host, __ATOMIC_RELAXED);
-        if (w2 == w) return CLOWNS_EHIP;  // unreachable: the device sets done at itermax
+        if (w2 == w) return CLOWNS_EHIP;  // unreachable
     }
     HIPCHK(hipMemcpyAsync(h->h_sc + sc_index, scal(seen + 1), sizeof(Scal), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -2240,7 +2246,7 @@ extern "C" int clowns_solver_create(clowns_solver **out, int device, void *strea
                     if (k.small < 0) k.small = 0;
                 }
         flag("CLOWNS_CLASSIFY_HOST", h->cls_force_host);
-        if (const char *e = getenv("CLOWNS_POLL")) h->poll = std::max(1, atoi(e));
+        if (const char *e = getenv("CLOWNS_POLL")) h->poll = std::min(QUEUE_MAX, std::max(QUEUE_MIN, atoi(e)));
         if (const char *e = getenv("CLOWNS_TAU_MIN")) h->tau_min = std::max(1e-8, atof(e));
         if (const char *e = getenv("CLOWNS_WILL_MAX_ROUNDS")) h->will_max_rounds = std::max(1, atoi(e));
     }
