@@ -1129,16 +1129,16 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
     // about geometrically), and h->poll at the least: the ones queued past the
     // end run out for nothing, which 8 to 16 at the end of each inner solve of a
     // mixed one made 4% of a time step.
-    int K = 1, seen = 0;
-    const int last = itermax + 1;  // whose first kernel posts the last iteration's word
+    long K = 1, seen = 0;
+    const long last = (long)itermax + 1;  // whose first kernel posts the last iteration's word
     bool done = itermax <= 0;  // PCGPME_WILL may ask for none
     int spins = 0, ahead = h->poll;
     while (!done) {
-        const int k0 = K;
-        while (K <= last && K - 1 - seen < ahead) iteration(K++);
+        const long k0 = K;
+        while (K <= last && K - 1 - seen < ahead) iteration((int)K++);
         if (K != k0) HIPCHK(hipGetLastError());
         const unsigned long long w = __atomic_load_n(host, __ATOMIC_RELAXED);
-        const int k = (int)(w >> 33);
+        const long k = (long)(w >> 33);
         done = (w >> 32 & 1) != 0;
         if (done || k != seen) {
             seen = k;
@@ -1146,7 +1146,7 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
             const unsigned bits = (unsigned)w;
             float e;
             std::memcpy(&e, &bits, sizeof(e));
-            const double rate = k > 0 ? -std::log((double)e) / k : 0.0;  // ERR starts at 1
+            const double rate = k > 0 ? -std::log((double)e) / (double)k : 0.0;  // ERR starts at 1
             const double left = rate > 0.0 && eps > 0.0 ? std::log(e / eps) / rate : 0.0;  // iterations to go
             ahead = left > 4.0 * QUEUE_MAX ? QUEUE_MAX : std::max(h->poll, left > 0.0 ? (int)(left / 4.0) : 0);
             continue;
@@ -1165,7 +1165,7 @@ int run_bicgstab(clowns_solver *h, const Op<T> &A, VecSet<T> &V, Scal *sc, int i
         const unsigned long long w2 = __atomic_load_n(host, __ATOMIC_RELAXED);
         if (w2 == w) return CLOWNS_EHIP;  // unreachable
     }
-    HIPCHK(hipMemcpyAsync(h->h_sc + sc_index, scal(seen + 1), sizeof(Scal), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(h->h_sc + sc_index, scal((int)(seen + 1)), sizeof(Scal), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     if (pf) {
         pf->kout.push_back(h->h_sc[sc_index].kout);
