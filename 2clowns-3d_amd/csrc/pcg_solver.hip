@@ -65,6 +65,7 @@ template <typename T> struct DevBuf {
         n = 0;
         hipError_t e = hipMalloc((void **)&p, std::max<size_t>(want, 1) * sizeof(T));
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by a later call's look at the last error
             p = nullptr;
             return e == hipErrorOutOfMemory ? CLOWNS_ENOMEM : CLOWNS_EHIP;
         }
@@ -93,6 +94,7 @@ template <typename T> struct VecSet {
     int ensure(size_t n) {
         DevBuf<T> *all[] = {&r, &rh, &p0, &q, &e, &v, &y, &t, &x};
         for (auto *b : all) {
+            if (b->n < n) padN = -1;  // new memory, also where a later vector finds none
             int rc = b->ensure(n);
             if (rc) return rc;
         }
@@ -1473,6 +1475,7 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     const int ldu = lda;
     lda = (N + 63) & ~63;
     const size_t nm = (size_t)lda * NL;
+    h->N = 0;  // no operator until the new one stands: a failed load leaves none
     if ((rc = h->AL.ensure(nm + RUN_PAD)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure((size_t)N + RUN_PAD)) ||
         (rc = h->W.ensure(N)))
         return rc;
@@ -1504,10 +1507,7 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     int hbad = 0;
     HIPCHK(hipMemcpyAsync(&hbad, h->flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    if (hbad) {
-        h->N = 0;
-        return CLOWNS_EBADARG;
-    }
+    if (hbad) return CLOWNS_EBADARG;
     double P1 = parm, P2;
     if (parm < 1.0) P1 = 2.0 * 2.0;
     P2 = P1 + 1.0;
@@ -1527,7 +1527,8 @@ int load_matrix(clowns_solver *h, const double *AL, int NL, int lda, const int *
     h->will_rev_valid = false;
     h->order_G = 0;  // a caller's operator: natural order unless set_block_order
     h->order_pending = false;
-    return build_forms(h);
+    if ((rc = build_forms(h))) h->N = 0;
+    return rc;
 }
 
 // Whether the small kernels run the resident operator in this precision: with
@@ -1810,24 +1811,22 @@ int build_runs(clowns_solver *h) {
         fprintf(stderr, "clowns_pcg: N=%d row runs: %d tasks, %d with their own coefficients, %d rows listed, "
                         "%d records\n", N, res[2], res[3], res[0], res[1]);
     if (res[0] > lcap) return CLOWNS_OK;
-    h->run_ok = true;
     h->run_dot = dot && res[1] <= rcap;
-    return pack_runs<double, double>(h, nullptr, h->run_pair, h->run_spmv, h->run_wave);
+    rc = pack_runs<double, double>(h, nullptr, h->run_pair, h->run_spmv, h->run_wave);
+    h->run_ok = rc == CLOWNS_OK;
+    return rc;
 }
 // What the kernels read of the resident operator beside its columns: the row
-// patterns, then the row runs, or the index codes of the column kernels.
+// patterns, then the row runs, or the index codes of the column kernels.  What
+// the operator before had is off from the start, so that a return in between
+// leaves no codes or tasks of another operator.
 int build_forms(clowns_solver *h) {
     int rc;
-    h->small64.ok = false;
-    if (small_size<double>(h)) {
-        if ((rc = build_small<double, double>(h, h->small64, h->AL.p, h->LL.p))) return rc;
-        h->pat_ok = h->run_ok = h->ll16_ok = h->ll8_ok = false;
-        h->pat_rows = 0;
-        return CLOWNS_OK;
-    }
+    h->small64.ok = h->small32.ok = h->smallt.ok = false;
+    h->pat_ok = h->run_ok = h->run_dot = h->ll16_ok = h->ll8_ok = h->t16_ok = h->t8_ok = false;
+    h->ll16_wide = h->ll8_wide = h->pat_rows = 0;
+    if (small_size<double>(h)) return build_small<double, double>(h, h->small64, h->AL.p, h->LL.p);
     if ((rc = build_patterns(h)) || (rc = build_runs(h))) return rc;
-    h->ll16_ok = h->ll8_ok = false;
-    h->ll16_wide = h->ll8_wide = 0;
     return h->run_ok && h->run_dot ? CLOWNS_OK : build_ll16(h);
 }
 // The FP32 forms (ensure_f32).
@@ -1982,8 +1981,8 @@ template <typename T> int ensure_vecs(clowns_solver *h, VecSet<T> &V, int N) {
 // single kernels run.
 template <typename T> int ensure_small(clowns_solver *h, VecSet<T> &V, Op<T> &A) {
     if (!A.small_G) return CLOWNS_OK;
+    if (V.p1.n < (size_t)A.N + VEC_PAD) V.padP1 = -1;
     if (V.p1.ensure((size_t)A.N + VEC_PAD) || h->small_part.ensure(16 * (size_t)geo_of(A.N, 2).G)) {
-        (void)hipGetLastError();
         A.small = {};
         A.small_G = 0;
         return CLOWNS_OK;
@@ -1998,6 +1997,7 @@ template <typename T> int ensure_small(clowns_solver *h, VecSet<T> &V, Op<T> &A)
 // The scaled right-hand side of a run (the mixed solve gathers it in its
 // first PM application): N + 64 entries, ghost rows zero.
 int ensure_bs(clowns_solver *h, int N) {
+    if (h->bs.n < (size_t)N + VEC_PAD) h->bs_padN = -1;
     int rc = h->bs.ensure((size_t)N + VEC_PAD);
     if (rc) return rc;
     if (h->bs_padN != N) {
@@ -2890,13 +2890,8 @@ int ensure_transpose(clowns_solver *h) {
     else
         k_scale_sort<4><<<cdiv(N, BS), BS, 0, s>>>(N, lda, h->ALt.p, h->LLt.p, h->Dt.p, h->Wt.p, P1, P2);
     HIPCHK(hipGetLastError());
-    h->smallt.ok = false;
-    if (h->small64.ok) {
-        h->t16_ok = h->t8_ok = false;
-        if ((rc = build_small<double, double>(h, h->smallt, h->ALt.p, h->LLt.p))) return rc;
-    } else if ((rc = build_codes_t(h))) {
-        return rc;
-    }
+    h->smallt.ok = h->t16_ok = h->t8_ok = false;
+    if ((rc = h->small64.ok ? build_small<double, double>(h, h->smallt, h->ALt.p, h->LLt.p) : build_codes_t(h))) return rc;
     h->have_t = true;
     return CLOWNS_OK;
 }
@@ -3063,6 +3058,7 @@ extern "C" int clowns_solver_assemble(clowns_solver *h, const clowns_grid_dev *g
     const int N = g->nrows;
     const int lda = (N + 63) & ~63;
     const size_t nm = (size_t)lda * 6;
+    h->N = 0;  // as load_matrix
     if ((rc = h->AL.ensure(nm + RUN_PAD)) || (rc = h->LL.ensure(nm)) || (rc = h->D.ensure((size_t)N + RUN_PAD)) ||
         (rc = h->W.ensure(N)))
         return rc;
@@ -3086,8 +3082,10 @@ extern "C" int clowns_solver_assemble(clowns_solver *h, const clowns_grid_dev *g
     h->have_t = false;
     h->raw_valid = keep_raw != 0;
     h->will_rev_valid = false;
-    if ((rc = build_forms(h))) return rc;
-    if ((rc = note_block_order(h, g))) return rc;
+    if ((rc = build_forms(h)) || (rc = note_block_order(h, g))) {
+        h->N = 0;
+        return rc;
+    }
     HIPCHK(hipStreamSynchronize(s));
     return CLOWNS_OK;
 }

@@ -81,7 +81,9 @@ int clowns_solver_set_stream(clowns_solver *h, void *stream);
 /* Load the operator from device arrays in the reference layout (AL/LL with
  * column stride lda >= N, LL 1-based, D length N).  Scales and sorts a copy
  * on the device (pcgpme_para.F90:77-112); the caller's arrays are not
- * modified.  The scaled/sorted matrix stays resident until the next call. */
+ * modified.  The scaled/sorted matrix stays resident until the next call; a
+ * call that fails once it has begun (memory, a neighbour index out of range)
+ * leaves none, and solves then return CLOWNS_EBADARG. */
 int clowns_solver_set_matrix(clowns_solver *h, const double *d_AL, int32_t NL,
                              int32_t lda, const int32_t *d_LL,
                              const double *d_D, int32_t N, double parm);
