@@ -339,7 +339,7 @@ struct clowns_solver {
     DevBuf<double> run_rc;
     DevBuf<float> run_rc32;
     int run_lcap = 0, run_nl = 0, run_nr = 0, run_nt[2] = {0, 0};
-    bool run_ok = false;
+    bool run_ok = false, run32_ok = false;  // FP64; the FP32 forms (ensure_f32)
     bool run_dot = false;         // described for k_pm_dot_run
     int pat_adj = 0;              // pattern rows whose last two slots are adjacent rows or ghosts
     DevBuf<float> AL32, D32;
@@ -1181,6 +1181,7 @@ int check_nl(int NL) { return (NL == 6 || NL == 4) ? CLOWNS_OK : CLOWNS_EBADNL; 
 
 int build_forms(clowns_solver *h);
 int build_runs32(clowns_solver *h);
+void release_runs32(clowns_solver *h);
 int order_runs(clowns_solver *h);
 int ensure_block_order(clowns_solver *h);
 
@@ -1580,12 +1581,16 @@ int ensure_f32(clowns_solver *h) {
     }
     h->have_h = h->kn.pm_half;
     h->have_rows = h->have_rows8 = false;
-    if ((rc = build_runs32(h))) return rc;
+    // as build_forms: without memory for the runs or the records the column kernels do
+    rc = build_runs32(h);
+    if (rc == CLOWNS_ENOMEM) release_runs32(h);
+    else if (rc) return rc;
     h->small32.ok = false;
-    if (small_size<float>(h) && !h->run_ok &&
-        (rc = h->have_h ? build_small<float, _Float16>(h, h->small32, h->ALh.p, h->LL.p)
-                        : build_small<float, float>(h, h->small32, h->AL32.p, h->LL.p)))
-        return rc;
+    if (small_size<float>(h) && !h->run_ok) {
+        rc = h->have_h ? build_small<float, _Float16>(h, h->small32, h->ALh.p, h->LL.p)
+                       : build_small<float, float>(h, h->small32, h->AL32.p, h->LL.p);
+        if (rc && rc != CLOWNS_ENOMEM) return rc;
+    }
     if (h->kn.rows32 && h->NL == 6 && h->ll16_ok && !h->run_ok) {
         const size_t n6 = (size_t)6 * h->N;
         if ((rc = h->ALr32.ensure(n6)) || (rc = h->Lr16.ensure(n6)) || (rc = h->nonunit.ensure(1))) return rc;
@@ -1816,21 +1821,43 @@ int build_runs(clowns_solver *h) {
     h->run_ok = rc == CLOWNS_OK;
     return rc;
 }
+// The runs' memory given back (that of their FP32 forms).
+void release_runs32(clowns_solver *h) {
+    for (auto &b : h->run_pair32) b.release();
+    h->run_spmv32.release(); h->run_c32.release(); h->run_wave32.release(); h->run_rc32.release();
+    h->run32_ok = false;
+}
+void release_runs(clowns_solver *h) {
+    release_runs32(h);
+    for (auto &b : h->run_raw) b.release();
+    for (auto &b : h->run_pair) b.release();
+    h->run_n.release(); h->run_raws.release(); h->run_spmv.release(); h->run_lj.release(); h->run_c.release();
+    h->run_cid.release(); h->run_rq.release(); h->run_wave.release(); h->run_rj.release(); h->run_rc.release();
+    h->run_ok = h->run_dot = false;
+}
 // What the kernels read of the resident operator beside its columns: the row
 // patterns, then the row runs, or the index codes of the column kernels.  What
 // the operator before had is off from the start, so that a return in between
-// leaves no codes or tasks of another operator.
+// leaves no codes or tasks of another operator; records and runs, without
+// which the column kernels do, are left out where there is no memory for them.
 int build_forms(clowns_solver *h) {
     int rc;
     h->small64.ok = h->small32.ok = h->smallt.ok = false;
-    h->pat_ok = h->run_ok = h->run_dot = h->ll16_ok = h->ll8_ok = h->t16_ok = h->t8_ok = false;
+    h->pat_ok = h->run_ok = h->run32_ok = h->run_dot = h->ll16_ok = h->ll8_ok = h->t16_ok = h->t8_ok = false;
     h->ll16_wide = h->ll8_wide = h->pat_rows = 0;
-    if (small_size<double>(h)) return build_small<double, double>(h, h->small64, h->AL.p, h->LL.p);
-    if ((rc = build_patterns(h)) || (rc = build_runs(h))) return rc;
+    if (small_size<double>(h)) {
+        rc = build_small<double, double>(h, h->small64, h->AL.p, h->LL.p);
+        if (rc != CLOWNS_ENOMEM) return rc;
+    }
+    if ((rc = build_patterns(h))) return rc;
+    rc = build_runs(h);
+    if (rc == CLOWNS_ENOMEM) release_runs(h);
+    else if (rc) return rc;
     return h->run_ok && h->run_dot ? CLOWNS_OK : build_ll16(h);
 }
 // The FP32 forms (ensure_f32).
 int build_runs32(clowns_solver *h) {
+    h->run32_ok = false;
     if (!h->run_ok) return CLOWNS_OK;
     const size_t nlc = RUN_LC * (size_t)h->run_lcap, nr = h->run_dot ? h->run_nr : 0;
     int rc;
@@ -1849,6 +1876,7 @@ int build_runs32(clowns_solver *h) {
     };
     h->kn.pm_half ? pm(k_run_list32<_Float16>) : pm(k_run_list32<float>);
     HIPCHK(hipGetLastError());
+    h->run32_ok = true;
     return CLOWNS_OK;
 }
 // The FP64 tasks in the operator's block order, once it is known (order_G set).
@@ -1857,7 +1885,7 @@ int order_runs(clowns_solver *h) {
     return pack_runs<double, double>(h, h->order.p, h->run_pair, h->run_spmv, h->run_wave);
 }
 template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
-    if (!h->run_ok) return;
+    if (!(sizeof(T) == 8 ? h->run_ok : h->have32 && h->run32_ok)) return;
     RunOp<T> &d = A.run;
     const size_t lcap = h->run_lcap;
     if constexpr (sizeof(T) == 8) {
@@ -1867,7 +1895,6 @@ template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
         d.sc = d.lc = h->run_c.p;
         d.rc = h->run_rc.p;
     } else {
-        if (!h->have32) return;
         d.pair[0] = h->run_pair32[0].p;
         d.pair[1] = h->run_pair32[1].p;
         d.spmv = h->run_spmv32.p;
@@ -2081,7 +2108,7 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
     Op<double> A = A_in;
     Op<float> A32 = A32_in;
     if ((rc = ensure_small(h, F, A32))) return rc;
-    const bool t64 = !A.run.spmv && !A.small.p01, t32 = !A.run.spmv && !A32.small.p01;
+    const bool t64 = !A.run.spmv && !A.small.p01, t32 = !A32.run.spmv && !A32.small.p01;
     if (t64) A.fuse = tune_fuse(h, A, V);
     if (t32) A32.fuse = tune_fuse(h, A32, F);
     if (t64) tune_stream(h, A, V);
@@ -2261,7 +2288,7 @@ extern "C" int clowns_solver_destroy(clowns_solver *h) {
     h->AL.release(); h->D.release(); h->W.release(); h->LL.release(); h->LL16.release(); h->base16.release(); h->LL8.release(); h->base8.release(); h->order.release(); h->order_first.release();
     h->AL32.release(); h->D32.release(); h->ALh.release(); h->ALr32.release(); h->Lr16.release(); h->Lr8.release(); h->nonunit.release(); h->pid.release(); h->ptab.release();
     h->small64.mem.release(); h->small32.mem.release(); h->smallt.mem.release(); h->small_part.release();
-    h->run_n.release(); h->run_raw[0].release(); h->run_raw[1].release(); h->run_raws.release(); h->run_pair[0].release(); h->run_pair[1].release(); h->run_spmv.release(); h->run_pair32[0].release(); h->run_pair32[1].release(); h->run_spmv32.release(); h->run_lj.release(); h->run_c.release(); h->run_c32.release(); h->run_cid.release(); h->run_rq.release(); h->run_wave.release(); h->run_wave32.release(); h->run_rj.release(); h->run_rc.release(); h->run_rc32.release();
+    release_runs(h);
     h->pat_keys.release();
     h->ALt.release(); h->Dt.release(); h->Wt.release(); h->LLt.release();
     h->LLt16.release(); h->baset16.release(); h->LLt8.release(); h->baset8.release();
@@ -2891,7 +2918,9 @@ int ensure_transpose(clowns_solver *h) {
         k_scale_sort<4><<<cdiv(N, BS), BS, 0, s>>>(N, lda, h->ALt.p, h->LLt.p, h->Dt.p, h->Wt.p, P1, P2);
     HIPCHK(hipGetLastError());
     h->smallt.ok = h->t16_ok = h->t8_ok = false;
-    if ((rc = h->small64.ok ? build_small<double, double>(h, h->smallt, h->ALt.p, h->LLt.p) : build_codes_t(h))) return rc;
+    rc = h->small64.ok ? build_small<double, double>(h, h->smallt, h->ALt.p, h->LLt.p) : CLOWNS_ENOMEM;
+    if (rc && rc != CLOWNS_ENOMEM) return rc;
+    if (!h->smallt.ok && (rc = build_codes_t(h))) return rc;
     h->have_t = true;
     return CLOWNS_OK;
 }
@@ -3477,9 +3506,11 @@ extern "C" int clowns_solver_tuning(clowns_solver *h, int32_t out[8]) {
     if (h->run_ok) {  // row runs: nothing is timed
         out[0] = out[1] = out[6] = 1;
         out[2] = op64(h).st_pm;
-        out[3] = h->have32 ? (int)op32(h).st_pm : -1;
-        out[4] = out[5] = 0;
-        out[7] = h->have32 ? 8 : -1;
+        const bool r32 = h->have32 && h->run32_ok;
+        out[3] = r32 ? (int)op32(h).st_pm : -1;
+        out[4] = 0;
+        out[5] = !h->have32 || r32 ? 0 : (h->ll16_ok ? 16 : 32);
+        out[7] = r32 ? 8 : -1;
         return CLOWNS_OK;
     }
     int f[2] = {-1, -1};
