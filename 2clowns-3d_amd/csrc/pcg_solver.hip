@@ -1620,7 +1620,7 @@ int build_ll16(clowns_solver *h) {
     // them
     const bool k64 = h->ix64 == 0 && tuned_size(h->N, h->ix64_N) && h->st64_f == force_key(h);
     const bool k32 = h->ix32 == 0 && tuned_size(h->N, h->ix32_N) && h->st32_f == force_key(h);
-    const bool want8 = h->kn.ll8 != 0 && !(h->kn.ll8 < 0 && k64 && k32);
+    const bool want8 = h->kn.ll8 == 1 || (h->kn.ll8 < 0 && !h->run_ok && !(k64 && k32));  // runs: RUN_PAT_ROWS
     int rc;
     if ((rc = h->LL16.ensure(nm)) || (rc = h->base16.ensure(nblk)) || (rc = h->flag.ensure(4))) return rc;
     if (want8 && ((rc = h->LL8.ensure(nm)) || (rc = h->base8.ensure(nblk8)))) return rc;
@@ -1757,6 +1757,15 @@ int pack_runs(clowns_solver *h, const int *order, DevBuf<RunPair<T>> *pair, DevB
 // against runs, 6.6/6.7 ms at 0.46M rows, 9.3/9.4 at 0.72M, 10.2/9.6 at 1.04M,
 // 15.6/13.0 at 1.65M; mixed 11.3/11.5 at 0.72M, 13.9/13.1 at 1.2M).
 constexpr int RUN_MIN_ROWS = 3 << 18;
+// Operators in runs whose last two slots are not the adjacent rows (a grid
+// whose spacing is not widest in x) have stage 5/6 by the column kernels: with
+// 16-bit codes (8-bit ones gain less than their build costs an assembly: 219.3
+// against 221.5 ms an FP64 step at 13.1M rows but 29.9 against 30.2 at 2.5M and
+// nothing mixed; 0.34 and 0.07 ms to build), in FP64 as k_pm_p2 from this size
+// on (off/on, ms an FP64 step: 17.6/17.9 at 1.18M rows, 21.3/21.7 at 1.66M,
+// 26.2/26.5 at 2.22M; 30.2/29.4 at 2.53M, 41.3/40.2 at 2.72M, 56.7/56.7 at
+// 4.34M, 221.5/215.7 at 13.1M).
+constexpr int RUN_PAT_ROWS = 9 << 18;
 
 // The row runs of the resident operator (with row patterns): used while the
 // lists hold at most an eighth of the rows (a listed row costs about as much
@@ -1814,7 +1823,8 @@ int build_runs(clowns_solver *h) {
     h->run_nt[1] = res[3];
     if (h->kn.verbose)
         fprintf(stderr, "clowns_pcg: N=%d row runs: %d tasks, %d with their own coefficients, %d rows listed, "
-                        "%d records\n", N, res[2], res[3], res[0], res[1]);
+                        "%d records, stage 5/6 by %s\n", N, res[2], res[3], res[0], res[1],
+                dot && res[1] <= rcap ? "runs" : "columns");
     if (res[0] > lcap) return CLOWNS_OK;
     h->run_dot = dot && res[1] <= rcap;
     rc = pack_runs<double, double>(h, nullptr, h->run_pair, h->run_spmv, h->run_wave);
@@ -1924,6 +1934,10 @@ template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
     // 157.5/156.3 at 19.5M, 240/232 at 30.4M, but 131.5/134.4 at 13.1M).  The
     // SpMV gained nothing from it (88.2 against 88.4 us at 13.1M).
     A.st_pm = (size_t)h->N * 3 * sizeof(T) > ((size_t)192 << 20);
+    if (!h->run_dot) {  // stage 5/6
+        A.pc2 = can_pc2(A) && (h->kn.pm_pat >= 0 ? h->kn.pm_pat == 1 : h->N >= RUN_PAT_ROWS);
+        A.ix8 = can_ix8(A);
+    }
 }
 
 // Views of the resident operator.
