@@ -1933,7 +1933,7 @@ template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
     // 110.2/107.9 at 12.2M, 449/436 at 24.3M, but 41.7/42.0 at 7.4M; FP32:
     // 157.5/156.3 at 19.5M, 240/232 at 30.4M, but 131.5/134.4 at 13.1M).  The
     // SpMV gained nothing from it (88.2 against 88.4 us at 13.1M).
-    A.st_pm = (size_t)h->N * 3 * sizeof(T) > ((size_t)192 << 20);
+    A.st_pm = h->kn.stream >= 0 ? (h->kn.stream & 1) != 0 : (size_t)h->N * 3 * sizeof(T) > ((size_t)192 << 20);
     if (!h->run_dot) {  // stage 5/6
         A.pc2 = can_pc2(A) && (h->kn.pm_pat >= 0 ? h->kn.pm_pat == 1 : h->N >= RUN_PAT_ROWS);
         A.ix8 = can_ix8(A);

@@ -74,3 +74,88 @@ def test_spacings(bed, scale, capfd):
             assert all(r[2] == 0 for r in ref)
         else:
             _same(got, ref)
+
+
+def _orders(N):
+    """The natural order of the 512-row blocks, a permutation, and back."""
+    import torch
+    G = ((N + 511) // 512 + 7) // 8 * 8
+    perm = np.random.default_rng(N).permutation(G).astype(np.int32)
+    return [None, torch.from_numpy(perm).to("cuda:0"), None]
+
+
+@pytest.mark.parametrize("stream", ["0", "1"], ids=["cached", "streamed"])
+@pytest.mark.parametrize("scale", [(1, 0.8, 1), (1, 1.25, 1)], ids=["runs", "columns"])
+def test_streams_and_block_orders(scale, stream):
+    dg = _grid("wavy", scale)
+    sol = _solver({"CLOWNS_RUNS": "0", "CLOWNS_STREAM": stream})
+    ref = _solve(sol, dg.assemble_into(sol), eps=1e-10, maxiter=4000)
+    sol.close()
+    sol = _solver({"CLOWNS_RUNS": "1", "CLOWNS_STREAM": stream})
+    b = dg.assemble_into(sol)
+    for order in _orders(dg.N):
+        sol.set_block_order(order)
+        _same(_solve(sol, b, eps=1e-10, maxiter=4000), ref)
+        t = sol.tuning()
+        assert t["index64"] == 0 and t["stream64"] == t["stream32"] == int(stream)
+    sol.close()
+
+
+def _arrays(N, adjacent, ghost):
+    """Runs of every kind (test_gpu_runs.synthetic), coefficients `ghost` on the
+    slots that have no neighbour."""
+    import torch
+    from test_gpu_runs import synthetic
+    LL, coef, D = synthetic(N, 11, 0.05, 0.0005, adjacent, 600)
+    coef = np.where(LL == 0, ghost, coef)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    return t(coef.T), t(LL.T), t(D)
+
+
+@pytest.mark.parametrize("adjacent", [True, False], ids=["adjacent", "not-adjacent"])
+def test_ghost_coefficients_orders_and_exits(adjacent):
+    """Ghost slots stay zero whatever their coefficient; a zero and a non-finite
+    right-hand side end a run at once, as by the column kernels."""
+    import torch
+    N = 262657
+    op = _arrays(N, adjacent, -0.01)
+    rng = np.random.default_rng(5)
+    b = rng.uniform(-1.0, 1.0, size=N)
+    nan, inf = b.copy(), b.copy()
+    nan[N // 3] = np.nan
+    inf[N - 1] = np.inf
+    rhs = [torch.from_numpy(v).to("cuda:0") for v in (b, b * 1e300, np.zeros(N), nan, inf)]
+    out = []
+    for runs in "01":
+        sol = _solver({"CLOWNS_RUNS": runs})
+        sol.set_matrix(*op)
+        got = []
+        for order in _orders(N):
+            sol.set_block_order(order)
+            for v in rhs:
+                got += _solve(sol, v, eps=1e-9, maxiter=25)
+        assert (sol.tuning()["index64"] == 0) == (runs == "1")
+        sol.close()
+        out.append(got)
+    _same(out[1], out[0])
+    first = out[0][:2 * len(rhs)]
+    assert np.all(np.isfinite(first[0][0])) and first[0][1] > 1
+    assert first[2][2] == 4001 and first[4][1:] == (0, 0)
+
+
+@pytest.mark.parametrize("cfg,rows", [(2, 2449992), (3, 13066133)])
+def test_full_size_default(cfg, rows):
+    """The forms that the solver takes by default at full size, the grid's block
+    order among them, against the column kernels."""
+    from clowns3d import DeviceGrid, configs
+    dg = DeviceGrid(configs.CONFIGS[cfg]())
+    assert dg.N == rows
+    out = []
+    for env in ({}, {"CLOWNS_RUNS": "0"}):
+        sol = _solver(env)
+        b = dg.assemble_into(sol)
+        out.append(_solve(sol, b, eps=1e-10))
+        assert (sol.tuning()["index64"] == 0) == (env == {})
+        sol.close()
+    _same(out[0], out[1])
+    assert all(r[2] == 0 for r in out[0])
