@@ -1889,10 +1889,11 @@ int build_runs32(clowns_solver *h) {
     h->run32_ok = true;
     return CLOWNS_OK;
 }
-// The FP64 tasks in the operator's block order, once it is known (order_G set).
+// The FP64 tasks in the operator's block order (order_G 0: natural), after it changed.
 int order_runs(clowns_solver *h) {
-    if (!h->run_ok || h->order_G != geo_of(h->N, 2).G) return CLOWNS_OK;
-    return pack_runs<double, double>(h, h->order.p, h->run_pair, h->run_spmv, h->run_wave);
+    if (!h->run_ok) return CLOWNS_OK;
+    return pack_runs<double, double>(h, h->order_G == geo_of(h->N, 2).G ? h->order.p : nullptr, h->run_pair,
+                                     h->run_spmv, h->run_wave);
 }
 template <typename T> void use_runs(const clowns_solver *h, Op<T> &A) {
     if (!(sizeof(T) == 8 ? h->run_ok : h->have32 && h->run32_ok)) return;
@@ -3547,8 +3548,9 @@ extern "C" int clowns_solver_set_block_order(clowns_solver *h, const int32_t *d_
     if (rc) return rc;
     h->order_pending = false;  // the caller's order replaces the grid's
     if (!d_order || G == 0) {
+        const bool was = h->order_G > 0;
         h->order_G = 0;
-        return CLOWNS_OK;
+        return was ? order_runs(h) : CLOWNS_OK;
     }
     if (G != geo_of(h->N, 2).G) return CLOWNS_EBADARG;
     // a permutation of 0..G-1, checked on the host before any kernel uses it

@@ -159,3 +159,21 @@ def test_full_size_default(cfg, rows):
         sol.close()
     _same(out[0], out[1])
     assert all(r[2] == 0 for r in out[0])
+
+
+def test_natural_order_again():
+    """set_block_order(None) takes the tasks back too, not the index arrays
+    alone: the SpMV is as fast as before the order that slowed it."""
+    from clowns3d import DeviceGrid, configs
+    dg = DeviceGrid(configs.config2())
+    sol = _solver({"CLOWNS_BLOCK_ORDER": "0"})
+    dg.assemble_into(sol)
+    times = []
+    for order in _orders(dg.N):
+        sol.set_block_order(order)
+        times.append(min(sol.time_kernel(0, 50) for _ in range(3)))
+    sol.close()
+    print(times)
+    # (13.1, 17.6 and 17.6 us before, the last now as the first)
+    assert times[1] > 1.15 * times[0]
+    assert times[2] < 0.5 * (times[0] + times[1])
