@@ -3422,7 +3422,7 @@ int vof_run(clowns_solver *h, const clowns_grid_dev *g, const double *d_Fp, int3
         HIPCHK(hipEventSynchronize(h->ev1));
         return CLOWNS_OK;
     };
-    static_assert(VOF_ROUNDS >= 2 && VC_ROUND + VOF_ROUNDS - 1 <= VC_N, "a counter a round, the last one VC_PENDING");
+    static_assert(VOF_ROUNDS >= 2 && VC_ROUND + VOF_ROUNDS - 1 <= VC_SLID, "a counter a round, the last one VC_PENDING");
     for (int r = 1; r <= VOF_ROUNDS; ++r)
         eval(r, r > 1 ? VC_ROUND + r - 2 : -1, r < VOF_ROUNDS ? VC_ROUND + r - 1 : VC_PENDING);
     apply();

@@ -54,7 +54,6 @@ constexpr int RUN_GHOST = 1 << 30;  // offset of a ghost slot while a block is d
 enum : int {
     RF_FAR = 1,     // bf: the partner's slot s leads elsewhere than back to the row
     RF_GHOST = 2,   // the partner is a ghost row (its stage value is 0)
-    RF_OWN = 4,     // coefficients are the rows' own (the operator's columns)
     RF_K4 = 4, RF_K5 = 6  // bits of the classes of slots 4 and 5 (RK_*)
 };
 template <typename T> struct alignas(16) RunPair {  // stages s, s + 1
@@ -88,7 +87,7 @@ template <typename T> struct RunOp {
     const int4 *lj0, *lj1;        // {row, n0, n1, n2}, {n3, n4, n5, 0}
     const int2 *lj2;              // {f of slot 1, f of slot 3}
     const T *sc, *lc;             // list coefficients of the operator and of the preconditioner
-    const T *AL, *D;              // the operator's columns (tasks with RF_OWN)
+    const T *AL, *D;              // the operator's columns (tasks of the rows' own coefficients)
     const uint8_t *cid;           // two-term stage (null: not in this form)
     const RunWave *wave;
     const int2 *rj;               // records: neighbours of slots 4, 5 ...
@@ -131,7 +130,7 @@ __device__ __forceinline__ void run_bounds(const unsigned long long *heads, int 
 // One workgroup describes one block.  pid: the rows' pattern ids.  Rows run
 // together while the six offsets and the partners' repeat: first the runs of
 // one pattern (the row's and its partners'), then, over what is left, those of
-// any coefficients (RF_OWN).  List entries and records come from an atomic
+// any coefficients.  List entries and records come from an atomic
 // allocation (their place depends on the run, their contents do not; past lcap
 // and rcap none are written).  cnt: list entries, records << 32: one atomic a
 // block (the four counters of a first form, of which atomics on one address
@@ -295,11 +294,10 @@ k_run_build(int N, int lda, const double *__restrict__ AL, const double *__restr
             int b[6];
 #pragma unroll
             for (int s = 0; s < 6; ++s) b[s] = off[h][s] == RUN_GHOST ? N : a + off[h][s];
-            const int fl0 = own[h] ? RF_OWN : 0;
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 const int mo = off[h][2 * s + 1];
-                int fl = fl0, bf = a;
+                int fl = 0, bf = a;
                 double cm = 0.0;
                 if (mo == RUN_GHOST) {
                     fl |= RF_GHOST;
@@ -313,7 +311,7 @@ k_run_build(int N, int lda, const double *__restrict__ AL, const double *__restr
                 RunPair<double> p = {a, r, hi, fl, b[2 * s], b[2 * s + 1], bf, 0, c[2 * s], c[2 * s + 1], cm};
                 (s ? o.pair1 : o.pair0)[k] = p;
             }
-            RunSpmv<double> q = {a, r, hi, fl0 | run_class(off[h][4]) << RF_K4 | run_class(off[h][5]) << RF_K5,
+            RunSpmv<double> q = {a, r, hi, run_class(off[h][4]) << RF_K4 | run_class(off[h][5]) << RF_K5,
                                  {b[0], b[1], b[2], b[3], b[4], b[5]}, {c[0], c[1], c[2], c[3], c[4], c[5]}, D[r]};
             o.spmv[k] = q;
         } else {

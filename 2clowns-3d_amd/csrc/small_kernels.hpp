@@ -227,7 +227,7 @@ template <typename T> __device__ __forceinline__ T small_14(const SmallOp<T> &A,
 }
 
 // out = PM in, with the dots of k_pm_v2 / k_pm_v4 (DOT 1: (w,out); 2: those and
-// (out,out); 3: (out,out); 0 none) as wavefront partials, one a workgroup of 64 R
+// (out,out)) as wavefront partials, one a workgroup of 64 R
 // rows (R rows a thread of those kernels), gridDim.x an array.  One row a
 // thread.
 template <typename T, int DOT>
@@ -235,29 +235,26 @@ __global__ void __launch_bounds__(256)
 k_small_pm(const Scal *__restrict__ sc, int N, SmallOp<T> A, const T *__restrict__ in, T *__restrict__ out,
            const T *__restrict__ w, double *__restrict__ wp) {
     constexpr int R = sizeof(T) == 8 ? 2 : 4;
-    __shared__ double pr[DOT == 2 ? 2 : 1][64 * R];
+    __shared__ double pr[DOT][64 * R];
     const int done = sc->done;
     const int lb = logical_block(), t = threadIdx.x, i = lb * 64 * R + t;
     double s0 = 0.0, s1 = 0.0;
     if (i < N) {
         const SmallLast<T> q = A.p45[i];
-        T wi = T(0);
-        if (DOT == 1 || DOT == 2) wi = w[i];
+        const T wi = w[i];
         const T t4 = small_14(A, in, i), u0 = small_14(A, in, q.j0), u1 = small_14(A, in, q.j1);
         T r = t4 - q.c0 * u0;
         r = r - q.c1 * u1;
         if (!done) out[i] = r;
-        if (DOT == 1 || DOT == 2) s0 = (double)wi * (double)r;
-        if (DOT == 2) s1 = (double)r * (double)r;
-        if (DOT == 3) s0 = (double)r * (double)r;
+        s0 = (double)wi * (double)r;
+        s1 = (double)r * (double)r;
     }
-    if (DOT == 0) return;
     pr[0][t] = s0;
-    if (DOT == 2) pr[DOT == 2 ? 1 : 0][t] = s1;
+    if (DOT == 2) pr[DOT - 1][t] = s1;
     __syncthreads();
     if (t >= 64 || done) return;
 #pragma unroll
-    for (int a = 0; a < (DOT == 2 ? 2 : 1); ++a) {
+    for (int a = 0; a < DOT; ++a) {
         double s = 0.0;
 #pragma unroll
         for (int k = 0; k < R; ++k)
