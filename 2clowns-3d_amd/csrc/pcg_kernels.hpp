@@ -20,8 +20,8 @@
 //                  block, deterministic order
 // Layout: matrix columns are structure-of-arrays with column stride lda
 // (identical to the reference's AL(NA,NL)/LL(NA,NL)); LL stays 1-based, so a
-// gather reads x[LL-1]; every vector has N+64 entries whose last 64 (the
-// ghost rows N+1+mod(I,64), :80) are zero.
+// gather reads x[LL-1]; every vector has zero rows after its N (VEC_PAD of
+// them), of which the first 64 are the ghost rows N+1+mod(I,64) (:80).
 // Arithmetic: expressions keep the Fortran's left-to-right order; the
 // library is compiled with -ffp-contract=off so single FP64 kernels agree
 // bit for bit with the reference.  Reductions: per-thread sums in row order,

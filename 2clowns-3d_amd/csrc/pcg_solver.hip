@@ -90,7 +90,7 @@ template <typename T> struct VecSet {
     DevBuf<T> r, rh, p0, q, e, v, y, t, x;
     DevBuf<T> p1;  // the second P of the small kernels, padded like the others
     int padP1 = -1;
-    int padN = -1;  // the row count whose ghost rows [N, N+64) were last zeroed
+    int padN = -1;  // the row count whose rows [N, N + VEC_PAD) were last zeroed
     int ensure(size_t n) {
         DevBuf<T> *all[] = {&r, &rh, &p0, &q, &e, &v, &y, &t, &x};
         for (auto *b : all) {
@@ -1996,16 +1996,17 @@ Op<float> op32(const clowns_solver *h) {
     return A;
 }
 
-// Ghost rows [N, N+64) of every vector of a run read as zero, as the
-// reference's zeroed work arrays do (pcgpme_para.F90:59-75): a gather through
-// a padding slot (LL = 0 -> N+1+mod(I,64), :80) then adds AL * 0 even where a
-// caller's AL is not 0 there.  Rows past N keep whatever a larger earlier
-// solve left, so the ghost rows are cleared whenever N changes.  VEC_SLACK
-// entries more follow the ghost rows: the FP32 SpMV gathers a row pair's two
-// neighbours with one 8-byte load (k_spmv_rows32), which through the last
-// ghost row reads the entry after it (its value is not used: the second row
-// of that pair has another neighbour and loads it on its own).
-// The row-run kernels read up to RUN_PAD zero rows.
+// VEC_PAD rows after row N - 1 of every vector of a run read as zero.  The first
+// PAD are the ghost rows, zero as the reference's work arrays are
+// (pcgpme_para.F90:59-75): a gather through a padding slot (LL = 0 ->
+// N+1+mod(I,64), :80) then adds AL * 0 even where a caller's AL is not 0 there.
+// Rows past N keep whatever a larger earlier solve left, so they are cleared
+// whenever N changes.  The FP32 SpMV gathers a row pair's two neighbours with
+// one 8-byte load (k_spmv_rows32), which through the last ghost row reads up to
+// VEC_SLACK entries after it (not used: the second row of that pair has another
+// neighbour and loads it on its own).  The row-run kernels load up to RUN_PAD
+// rows past the last one, lanes that store nothing and ghost slots among them:
+// that their loads stay within the vectors rests on VEC_PAD.
 constexpr int VEC_SLACK = 4;
 constexpr int VEC_PAD = std::max(PAD + VEC_SLACK, RUN_PAD);
 template <typename T> int ensure_vecs(clowns_solver *h, VecSet<T> &V, int N) {
@@ -2037,7 +2038,7 @@ template <typename T> int ensure_small(clowns_solver *h, VecSet<T> &V, Op<T> &A)
 }
 
 // The scaled right-hand side of a run (the mixed solve gathers it in its
-// first PM application): N + 64 entries, ghost rows zero.
+// first PM application), zero rows after it as after the vectors.
 int ensure_bs(clowns_solver *h, int N) {
     if (h->bs.n < (size_t)N + VEC_PAD) h->bs_padN = -1;
     int rc = h->bs.ensure((size_t)N + VEC_PAD);
@@ -2361,9 +2362,9 @@ extern "C" int clowns_solver_solve(clowns_solver *h, const double *d_b, double *
 // ----------------------------------------------------- allocation-free solve
 // The work memory of clowns_solver_solve_noalloc: a file-scope device array
 // (every GPU the library runs on holds its own copy until the process ends)
-// for the runs' vectors (nine FP64 and nine FP32 ones of N + 64 entries and
-// their slack, each 256-byte aligned), the scaled right-hand side, the dot
-// partials and the run scalars, for up to NOALLOC_MAX_ROWS rows: 65 MiB.
+// for the runs' vectors (ten FP64 and ten FP32 ones of N + VEC_PAD entries,
+// each 256-byte aligned), the scaled right-hand side, the dot partials (the
+// small kernels' too) and the run scalars, for up to NOALLOC_MAX_ROWS rows: 65 MiB.
 constexpr int NOALLOC_MAX_ROWS = 1 << 19;
 constexpr size_t NA_VEC = (size_t)NOALLOC_MAX_ROWS + 704;                  // entries per vector
 constexpr size_t NA_G1 = (((size_t)NOALLOC_MAX_ROWS + BS - 1) / BS + 7) / 8 * 8;  // largest grid

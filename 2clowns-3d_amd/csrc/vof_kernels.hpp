@@ -59,9 +59,9 @@ __device__ __forceinline__ int vof_block() {
 // counters: [0] retry (cal_new_f's icon = 30), [1] stop (F > F_lim on a
 // surface cell), [2] correction aimed at a solid cell, [3] pending cells of
 // the last modify round, [4] corrected cells, [6] invalid flags, [8..] pending
-// cells of the first rounds, [16..] slid cells, in VC_SLOTS counters of a cache
-// line each: atomics on one address take their turns, some 50 ns each, which
-// cost k_vof_slide 8 us (a wavefront's count each)
+// cells of the first rounds, [16..] slid cells, in VC_SLOTS counters 64 bytes
+// apart (two to a cache line): atomics on one address take their turns, some 50
+// ns each, which cost k_vof_slide 8 us (a wavefront's count each)
 enum { VC_RETRY = 0, VC_STOP = 1, VC_SOLID = 2, VC_PENDING = 3, VC_MODIFIED = 4, VC_BAD = 6, VC_ROUND = 8,
        VC_SLID = 16, VC_SLOTS = 64, VC_LINE = 16, VC_N = VC_SLID + VC_SLOTS * VC_LINE };
 constexpr int VOF_ROUNDS = 2;  // modify rounds queued before the host looks

@@ -101,7 +101,7 @@ int clowns_solver_solve(clowns_solver *h, const double *d_b, double *d_x,
  * time-stepping loops, harnesses that forbid it).  No counterpart in the
  * reference.  Same arguments and results as clowns_solver_solve (bit for
  * bit); the run's work vectors, scaled right-hand side, dot partials and
- * scalars live in a file-scope device array of the library, 58 MiB, which
+ * scalars live in a file-scope device array of the library, 65 MiB, which
  * every GPU the library runs on holds until the process ends.  Limits: at
  * most 524288 rows (CLOWNS_EBADARG beyond, with a message on stderr); the
  * operator comes from clowns_solver_set_matrix / clowns_solver_assemble as
