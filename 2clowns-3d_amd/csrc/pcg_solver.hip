@@ -2050,6 +2050,16 @@ int ensure_bs(clowns_solver *h, int N) {
     return CLOWNS_OK;
 }
 
+// Waits for what a solve queued when it is left before its end, by an error:
+// kernels that were still to run would post their words into the next solve's.
+struct Drain {
+    hipStream_t s;
+    bool on = true;
+    ~Drain() {
+        if (on) (void)hipStreamSynchronize(s);
+    }
+};
+
 // FP64 PCGPME on the resident operator `A` with row scales `Wsc`: exactly the
 // reference's sequence (setup :115-145, iteration :148-247).
 // beta_prod selects PCGPME_WILL's rounding of BETA (pcgpme_2DH.f90:241).
@@ -2071,6 +2081,7 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
     const int G1 = geo_of(N, 1).G;
     Scal *sc = h->sc.p;
     double *part = h->part.p;
+    Drain drain{s};
     HIPCHK(hipEventRecord(h->ev0, s));
     k_reset<<<1, 64, 0, s>>>(sc, eps, itermax, beta_prod ? 1 : 0);
     // WK1 = W*B; X = x0.
@@ -2093,6 +2104,7 @@ int solve_fp64(clowns_solver *h, const Op<double> &A_in, const double *Wsc, cons
     HIPCHK(hipMemcpyAsync(d_x, V.x.p, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, s));
     HIPCHK(hipEventRecord(h->ev1, s));
     HIPCHK(hipStreamSynchronize(s));
+    drain.on = false;
     const Scal &hs = h->h_sc[0];
     if (info) {
         float ms = 0.f, ms0 = 0.f;
@@ -2134,6 +2146,7 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
     const int G1 = geo_of(N, 1).G;
     Scal *sc = h->sc.p, *outer = h->sc.p + 1;
     double *part = h->part.p;
+    Drain drain{s};
     HIPCHK(hipEventRecord(h->ev0, s));
     k_reset<<<1, 64, 0, s>>>(outer, eps, itermax, 0);
     k_reset<<<1, 64, 0, s>>>(sc, eps, itermax, 0);
@@ -2201,6 +2214,7 @@ int solve_mixed(clowns_solver *h, const Op<double> &A_in, const Op<float> &A32_i
     HIPCHK(hipMemcpyAsync(d_x, V.x.p, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, s));
     HIPCHK(hipEventRecord(h->ev1, s));
     HIPCHK(hipStreamSynchronize(s));
+    drain.on = false;
     if (info) {
         float ms = 0.f, ms0 = 0.f;
         (void)hipEventElapsedTime(&ms, h->ev0, h->ev1);

@@ -70,3 +70,40 @@ def test_largest_maxiter_dropin():
     print(out[0][0], out[1][0])
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("small", ["0", "1"], ids=["single-kernels", "five-launches"])
+def test_solve_after_one_left_by_an_error(small):
+    """A solve that an error ends (here one that the host program left behind)
+    waits for the kernels it had queued: while the GPU is still busy with other
+    work, their word that a zero right-hand side is done must not end the next
+    solve."""
+    import ctypes
+    import torch
+    from clowns3d import ClownsError, Solver
+    s = box_system(24, 16, 10, seed=3)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    os.environ["CLOWNS_SMALL"] = small
+    try:
+        sol = Solver(0)  # reads the switch at creation
+    finally:
+        del os.environ["CLOWNS_SMALL"]
+    sol.set_matrix(t(s["AL"].T), t(s["LL"].T), t(s["D"]))
+    b = t(s["B"])
+    zero, x0, x = torch.zeros_like(b), torch.zeros_like(b), torch.zeros_like(b)  # torch itself stops at such an error
+    ref, iref = sol.solve(b, eps=1e-10)
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    a = torch.ones((8192, 8192), device="cuda:0")
+    torch.cuda.synchronize()
+    for _ in range(20):
+        a @ a
+    assert hip.hipSetDevice(9999) != 0
+    with pytest.raises(ClownsError) as e:
+        sol.solve(zero, x0, eps=1e-10)
+    assert e.value.code == 4004
+    x, i = sol.solve(b, x, eps=1e-10)
+    torch.cuda.synchronize()
+    assert (i["iters"], i["ier"]) == (iref["iters"], 0) and torch.equal(x, ref)
+    sol.close()
