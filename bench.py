@@ -18,9 +18,10 @@ solve and against the FP64 solution, and its own roofline entry.
 roofline: one more step of each form with HIP events around every kernel
 launch on the solver's stream (clowns_solver_kernel_profile): the kernel
 class with the most in-solve time, its average launch duration and its
-algorithmic bytes per launch (CLASS_BYTES x rows); `traffic` from
-profiles/traffic_config<n>.json, written by --traffic from two rocprofv3
---pmc runs (FETCH_SIZE, WRITE_SIZE) of --pmc-run.
+algorithmic bytes per launch (CLASS_BYTES x rows: `achieved`, `frac`); `traffic`,
+the bytes it moves by the counters, from profiles/traffic_config<n>.json, written
+by --traffic from two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE) of
+--pmc-run, and the rate of these (`moved_GBps`, `moved_frac`).
 
 cpu_baseline: the reference's own PCGPME (flang build of pcgpme_para.F90,
 oracle/_ref) on the same system assembled on the host, run to convergence at
@@ -64,7 +65,9 @@ PEAK_HBM_GBS = 8000.0
 DESCR = {1: "wavy surface at 0.6H + 16x16x12 obstacle", 2: "wavy surface at 0.6H + 64x64x24 obstacle",
          3: "40 Gaussian bed bumps, partial cells fb in [0.05,1], wavy surface at 0.6H"}
 # Algorithmic bytes per matrix row (values and vectors each kernel must stream
-# once; index arrays excluded).  Whole iteration: 512 B/row at FP64.
+# once; index arrays excluded).  Whole iteration: 512 B/row at FP64.  They count
+# every row's coefficients, which the kernels by row runs hardly read (a pair of
+# stages moves 16 of its 32): a rate of these bytes may exceed the copy rate.
 ALG_BYTES = {
     "spmv": 72,        # AL 48 + D 8 + x 8 + y 8
     "pm_stage": 24,    # AL_j 8 + in 8 + out 8
@@ -612,9 +615,13 @@ CLASS_BYTES = {"spmv": 72, "pm_stage": 24, "pm_pair": 32, "pm_dot": 40, "p_updat
 
 def kernel_names(tune, precision):
     """Names of the kernel forms the solver runs on this operator, per class."""
-    if tune["index64" if precision == "fp64" else "index32"] == 0:  # row runs
-        T, c = ("double", "double") if precision == "fp64" else (
-            "float", "_Float16" if os.environ.get("CLOWNS_PM_HALF", "1") != "0" else "float")
+    T, c = ("double", "double") if precision == "fp64" else (
+        "float", "_Float16" if os.environ.get("CLOWNS_PM_HALF", "1") != "0" else "float")
+    index = tune["index64" if precision == "fp64" else "index32"]
+    if index < 0:  # no form was chosen between: an iteration in five launches
+        return {"spmv": f"k_small_spmv<{T},STEP,4>", "pm_dot": f"k_small_pm<{T},DOT>",
+                "xr_update": f"k_small_update<{T},4>"}
+    if index == 0:  # row runs
         st = "true" if tune["stream64" if precision == "fp64" else "stream32"] == 1 else "false"
         V = "vec<%s>" % T
         return {"spmv": f"k_spmv_run<{T},0>", "pm_pair": f"k_pm_pair_run<{T},S,{st},{c}>",
@@ -662,8 +669,11 @@ def dominant(prof, precision, N, tune, traffic):
     alg = CLASS_BYTES[cls] * scale * N
     name = kernel_names(tune, precision)[cls]
     achieved = alg / (avg_us * 1e-6) / 1e9
+    moved = (traffic or {}).get(name)
+    moved_gbs = moved / (avg_us * 1e-6) / 1e9 if moved else None
     out = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-           "frac": achieved / PEAK_HBM_GBS, "traffic": (traffic or {}).get(name), "kernel": name,
+           "frac": achieved / PEAK_HBM_GBS, "traffic": moved, "moved_GBps": moved_gbs,
+           "moved_frac": moved_gbs / PEAK_HBM_GBS if moved else None, "kernel": name,
            "kernel_class": cls, "launches": n, "avg_us": avg_us, "alg_bytes_per_launch": alg,
            "alg_bytes_per_row": CLASS_BYTES[cls] * scale,
            "in_solve_us": {c: round(v[1] * 1e3 / v[0], 2) for c, v in prof[precision].items() if v[0] > 0},
@@ -754,10 +764,16 @@ def _short_name(k):
     """rocprof's demangled kernel name in the form kernel_names uses:
     'void clowns::k_pm_v2<double, 1, 0, clowns::Ix8, true, double>(...)' ->
     'k_pm_v2<double,1,0,Ix8,true,double>' (the dot-carrying stages' DOT
-    argument becomes the word DOT)."""
+    argument becomes the word DOT, a pair's first stage S, a small SpMV's step
+    STEP)."""
     if k.startswith("_ZN6clowns"):
         k = _demangle_args(k)
     k = k.split("(")[0].replace("void ", "").replace("clowns::", "").replace(" ", "").strip()
+    for pre, word in (("k_pm_pair_run<", "S"), ("k_pm_dot_run<", "DOT"), ("k_small_pm<", "DOT"),
+                      ("k_small_spmv<", "STEP")):
+        if k.startswith(pre):
+            args = k[len(pre):-1].split(",")
+            return pre + ",".join([args[0], word] + args[2:]) + ">"
     for pre in ("k_pm_v2<double,2,", "k_pm_v4<2,", "k_pm_v4<1,", "k_pm_p2<2,", "k_pm_p2<1,"):
         if k.startswith(pre):
             rest = k[len(pre):]
@@ -864,15 +880,16 @@ def main():
         return info
 
     if args.pmc_run:
-        # an assembled FP64 solve and a mixed solve in each of the kernel
-        # forms the solver may pick here (streamed or cached PM stages and
+        # an assembled FP64 solve and a mixed solve in the default form and in
+        # each of the column kernels' forms (streamed or cached PM stages and
         # SpMV, 8- or 16-bit index codes, single or fused PM stages, FP64 PM
         # stages with or without the pattern table), so the traffic of
         # whichever form a timed run picks was counted inside a solve; then
         # the copy kernel the counters are scaled by
         tunes = []
-        for st, ll8, fuse, pat in itertools.product(("0", "1", "2", "3"), ("0", "1"), ("0", "1"), ("0", "1")):
-            env = {"CLOWNS_STREAM": st, "CLOWNS_LL8": ll8, "CLOWNS_FUSE_PM": fuse, "CLOWNS_PM_PAT": pat}
+        forms = [{}] + [{"CLOWNS_STREAM": st, "CLOWNS_LL8": ll8, "CLOWNS_FUSE_PM": fuse, "CLOWNS_PM_PAT": pat}
+                        for st, ll8, fuse, pat in itertools.product("0123", "01", "01", "01")]
+        for env in forms:
             os.environ.update(env)
             try:
                 s2 = Solver(0)
