@@ -562,7 +562,10 @@ struct RunGrid {
     int own, list, tab;
 };
 // At 12.2M rows (wavy bed): FP64 37.5 us, 5.2 TB/s of the vectors read and
-// written (k_pm2_v2: 93; two single stages: 79); FP32 26 (65; 51).
+// written (k_pm2_v2: 93; two single stages: 79); FP32 26 (65; 51).  At 13.1M rows
+// of a bathymetry 61 and 40 us: by the counters 23.0 and 12.9 bytes a row (16 and
+// 8 of them the vectors'), 4.9 and 4.2 TB/s, and 11 million L1 accesses where
+// k_pm2_v2 makes 33.
 template <typename T, int S, bool ST, typename C>
 __global__ void __launch_bounds__(BS)
 k_pm_pair_run(const Scal *__restrict__ sc, int N, const T *__restrict__ in, T *__restrict__ out, RunOp<T> d,
@@ -672,7 +675,8 @@ __device__ __forceinline__ void run_spmv_finish(int v, int o, RunVS<T> &w, const
 // y = A x (MODE 0) or y = v1 - A x (MODE 3), NL = 6.  At 12.2M rows (wavy bed):
 // FP64 55 us, 3.5 TB/s of x and y (k_spmv_v2: 78); FP32 32 (k_spmv_rows32: 46).
 // At 13.1M rows of a bathymetry 88 and 53 (105 and 76): its listed rows, 3% of
-// all, each fetch six cache lines of their own.
+// all, each fetch six cache lines of their own; 28.9 and 18.3 bytes a row by the
+// counters, 4.3 and 4.5 TB/s, and 17.6 million L1 accesses (k_spmv_v2: 33.5).
 template <typename T, int MODE>
 __global__ void __launch_bounds__(BS)
 k_spmv_run(const Scal *__restrict__ sc, int N, const T *__restrict__ x, const T *__restrict__ v1, T *__restrict__ y,
@@ -724,8 +728,9 @@ k_spmv_run(const Scal *__restrict__ sc, int N, const T *__restrict__ x, const T 
 // pattern table, whose row p lane p holds; rows with a record take theirs by
 // rank from the lane that loaded it, while the ids are still on their way (a
 // load by rank after them was a dependent trip more: 74.6 against 70.4 us).
-// FP64: block order as k_pm_v2's; FP32: natural.  What bounds it is HBM: 25
-// bytes a row, 4.7 TB/s at 13.1M rows (70 us; k_pm_p2 76; FP32 45, k_pm_v4 46).
+// FP64: block order as k_pm_v2's; FP32: natural.  What bounds it is HBM: 26.8
+// bytes a row by the counters (14.1 FP32), 5.1 TB/s at 13.1M rows (69 us; k_pm_p2
+// 76; FP32 44.5, 4.1 TB/s; k_pm_v4 46).
 template <typename T, int DOT, bool ST, typename C>
 __global__ void __launch_bounds__(BS)
 k_pm_dot_run(const Scal *__restrict__ sc, int N, const T *__restrict__ in, T *__restrict__ out,
